@@ -121,6 +121,31 @@ SADMC_HD double lj_pair(double r2) {
   return 4.0 * (s6 - s3);
 }
 
+// 1/x by the hardware reciprocal, two Newton steps and one residual
+// correction: the operations of the compiler's own 1.0 / x without its
+// operand scaling and special-case fix-up, so the same bits wherever those do
+// nothing (2^-766 < x < 2^766 at least).  Outside, the pair terms below are
+// the division's all the same: for smaller x both reciprocals exceed 2^765,
+// s^6 and s^3 overflow and the term is NaN; for larger finite x both have s^2
+// = 0 and the term is +0; only at +inf (and NaN) is the fast one NaN where the
+// division's may not be, which the pair loops test for.
+SADMC_DF double recip_f64_fast(double x) {
+  double y = __builtin_amdgcn_rcp(x);
+  y = __builtin_fma(y, __builtin_fma(-x, y, 1.0), y);
+  y = __builtin_fma(y, __builtin_fma(-x, y, 1.0), y);
+  return __builtin_fma(__builtin_fma(-x, y, 1.0), y, y);
+}
+
+// lj_pair with recip_f64_fast.
+SADMC_DF double lj_pair_fast(double r2) {
+  double s = recip_f64_fast(r2);
+  double s2 = s * s;
+  double s4 = s2 * s2;
+  double s6 = s2 * s4;
+  double s3 = s * s2;
+  return 4.0 * (s6 - s3);
+}
+
 // The same pair term in binary32 (precision variant).
 SADMC_HD float lj_pair_f32(float r2) {
   float s = 1.0f / r2;

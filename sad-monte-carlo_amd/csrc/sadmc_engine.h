@@ -41,18 +41,18 @@ struct PExtra {
   double total;
 };
 
-// Bin records are split by when they are needed.  The hot part (16 bytes)
-// is all the accept/reject decision reads; the cold part is read-modify-
-// written one move later, so its load overlaps the next move's pair sums.
-// WL's own histogram lives in a third array that only WL kernels touch.
+// Bin records are split by who reads them.  The hot part (16 bytes) is what
+// the accept/reject decision and the entropy reduction read; the cold part (32
+// bytes, so that no record straddles a cache line) is what a visit updates;
+// t_found is written on a bin's first visit only.  WL's own histogram lives
+// in another array that only WL kernels touch.
 struct HotBin {
   double lnw;
   uint64_t hist;
 };
-struct ColdBin {
+struct alignas(32) ColdBin {
   double etot, esq;
   uint64_t rt, vep;
-  uint64_t tfound, pad;
 };
 
 // Arguments of one walker set, passed by value to the kernels (they live in
@@ -63,6 +63,7 @@ struct SetArgs {
   uint64_t *spins;   // [W]
   HotBin *hot;       // [W][cap]
   ColdBin *cold;     // [W][cap]
+  uint64_t *tfound;  // [W][cap]
   uint64_t *wlh;     // [W][cap] WL histogram, or null
   PExtra *extra;     // [W][cap] (WCA pressure) or null
   int32_t *flag;     // set to 1 when any walker of the set stops with a status
@@ -111,14 +112,16 @@ __device__ __forceinline__ double group_sum(double v, int G) {
 
 // rand 0.7 UniformInt sampling with a precomputed zone (lj.rs:368 /
 // ising.rs:105 semantics; the zone is the only part that depends on n).
-__device__ __forceinline__ uint64_t sample_zone(uint64_t &s0, uint64_t &s1, uint64_t range, uint64_t zone) {
+// The range fits 32 bits, so the 128-bit product takes two 32 x 32 + 64
+// multiply-adds.
+__device__ __forceinline__ uint32_t sample_zone(uint64_t &s0, uint64_t &s1, uint32_t range, uint64_t zone) {
   for (;;) {
-    uint64_t v = rng_next(s0, s1);
-    uint64_t lo = v * range;
-    if (lo <= zone) return __umul64hi(v, range);
+    const uint64_t v = rng_next(s0, s1);
+    const uint64_t a = (uint64_t)(uint32_t)v * range;
+    const uint64_t b = (uint64_t)(uint32_t)(v >> 32) * range + (a >> 32);
+    if (((b << 32) | (uint32_t)a) <= zone) return (uint32_t)(b >> 32);
   }
 }
-
 
 
 // MV = 1: the learned Gaussian move with its Hastings term (LJ only).
@@ -132,7 +135,7 @@ struct Engine {
   HotBin *H;
   ColdBin *Cb;
   uint64_t *WH;
-  PExtra *X;
+  int wk;  // the walker's index in its set
   // system
   double *lx, *ly, *lz;
   // This lane's atoms in registers, or (kLdsPos) read from the LDS mirror:
@@ -148,8 +151,9 @@ struct Engine {
   // EnergyMC scalars
   uint64_t s0, s1;
   double E, err;
-  uint64_t moves, accepted;
-  double tm;  // (double)moves, kept exact by +1.0 steps
+  uint64_t accepted;
+  double tm;  // the move count, whole and exact (below 2^53)
+  SADMC_DF uint64_t moves() const { return (uint64_t)tm; }
   double acc_rate, tscale, usc;
   double bmin;
   int32_t base, len;
@@ -157,28 +161,30 @@ struct Engine {
   int32_t max_S_index;
   uint64_t epoch;
   int32_t bulk, status, method;
-  // SAD
-  double too_lo, too_hi, lam, min_T, tF_d, Ns_d, lnw_lo, lnw_hi;
-  uint64_t tL, tF, Ns, highest, tmax;
+  double btop;  // bmin + width * len, the upper edge of the bins
+  // SAD (tF and N_s are whole and exact); rtF, rNs = 1 / tF, 1 / N_s and
+  // gzero (gamma is 0) follow lam, tF and N_s, which change rarely; tl_now:
+  // tL was set in this move.  min_T, tL, the largest t_found and WCA's
+  // has_pressure are touched so rarely that they stay in the walker's record.
+  double too_lo, too_hi, lam, tF, Ns, rtF, rNs, lnw_hi;
+  bool gzero, tl_now;
+  uint64_t highest;
   int32_t ilo, ihi;
+  SADMC_DF sadmc_walker_state &rec() const { return args().ws[wk]; }
+  SADMC_DF uint64_t *tfound() const { return args().tfound + (int64_t)wk * args().cap; }
   // SAMC / WL
   double t0, wl_gamma, wl_Ns, wl_min_e;
   uint64_t wl_lowest, wl_highest, wl_total;
   int32_t wl_len;
-  int32_t has_pressure;
-  // current bin (logical cur_i, physical cur_p): hot record (and WL count)
+  // current bin (logical cur_i, physical cur_p): its whole record (and WL
+  // count), written back when the walker leaves the bin; cur_p = -1: none
   int32_t cur_i, cur_p;
   double c_lnw;
   uint64_t c_hist, c_wlh;
-  // cold record of bin kp, and the previous move's cold work on it
-  int32_t kp;
-  double k_etot, k_esq;
-  uint64_t k_rt, k_vep;
-  int32_t pend, pend_rt, pend_bulk;
-  double pend_E;
-  uint64_t pend_epoch;
+  double c_etot, c_esq;
+  uint64_t c_rt, c_vep;
   // periodic triggers
-  uint64_t next_check, next_press;
+  double next_check, next_press;  // in moves
   // pending move
   int32_t pw;
   double ptx, pty, ptz, pe, pdabse;
@@ -187,10 +193,9 @@ struct Engine {
   float *XC;
   double lnh;
   // this move's SAD gamma, computed while the proposed bin's record loads
-  // (valid unless the move changed lambda or N_s), and the next uniform with
+  // (again if the move changes lambda or N_s), and the next uniform with
   // the generator state after drawing it, computed before it is needed
   double gpre, spec_u;
-  bool gdirty;
   uint64_t spec0, spec1;
   // sqrt(1 / moves) for the group's next G moves: lane l holds the value of
   // move rs_first + l; rs_next counts the moves served from it (G = empty)
@@ -206,10 +211,9 @@ struct Engine {
     n = a.n;
     H = a.hot + (int64_t)walker * a.cap;
     Cb = a.cold + (int64_t)walker * a.cap;
-    WH = a.wlh ? a.wlh + (int64_t)walker * a.cap : nullptr;
-    X = a.extra ? a.extra + (int64_t)walker * a.cap : nullptr;
-    kp = -1;
-    pend = 0;
+    wk = walker;
+    WH = METH == M_WL ? a.wlh + (int64_t)walker * a.cap : nullptr;
+    cur_p = -1;
     if (SYS == SYS_ISING) {
       spins = a.spins[walker];
     } else {
@@ -243,8 +247,7 @@ struct Engine {
     s1 = w.rng[1];
     E = w.E;
     err = w.error;
-    moves = w.moves;
-    tm = (double)moves;
+    tm = (double)w.moves;
     rs_next = 1 << 30;
     accepted = w.accepted_moves;
     acc_rate = w.acceptance_rate;
@@ -262,12 +265,9 @@ struct Engine {
       too_lo = w.too_lo;
       too_hi = w.too_hi;
       lam = w.latest_parameter;
-      min_T = w.min_T;
-      tL = w.tL;
-      tF = w.tF;
-      Ns = w.num_states;
+      tF = (double)w.tF;
+      Ns = (double)w.num_states;
       highest = w.highest_hist;
-      tmax = w.tmax;
     }
     if (METH == M_SAMC || METH == M_WL) t0 = w.t0;
     if (METH == M_WL) {
@@ -279,15 +279,14 @@ struct Engine {
       wl_total = w.wl_total_hist;
       wl_len = (int32_t)w.wl_len;
     }
-    if (SYS == SYS_WCA) has_pressure = w.has_pressure;
     if (SYS != SYS_ISING) {
       if (SYS == SYS_LJ) R2 = w.geom * w.geom;
       L = w.geom;
       halfL = 0.5 * w.geom;
     }
-    tF_d = (double)tF;
-    Ns_d = (double)Ns;
     usc = SYS == SYS_ISING ? 0.0 : uniform_scale(-tscale, tscale);
+    btop = bmin + args().width * (double)len;
+    if (METH == M_SAD) gamma_changed();
     cur_p = -1;
     if (!status) {
       refresh_indices();
@@ -295,18 +294,41 @@ struct Engine {
     }
   }
 
-  // Write back the walker state; `all` also writes the fields a method
-  // family does not use (only from_params needs that).
-  SADMC_DF void store(int walker, bool all = false) {
-    apply_pending();
-    write_cold();
+  // Write back the walker state; the fields that only from_params sets, or
+  // that are kept in the record during a launch, are not here.
+  SADMC_DF void store(int walker) {
+    write_back();
+    if (lane == 0) {
+      sadmc_walker_state &w = args().ws[walker];
+      if (METH == M_SAD) {
+        w.too_lo = too_lo;
+        w.too_hi = too_hi;
+        w.latest_parameter = lam;
+        w.tF = (uint64_t)tF;
+        w.num_states = (uint64_t)Ns;
+        w.highest_hist = highest;
+      }
+      if (METH == M_SAMC || METH == M_WL) w.t0 = t0;
+      if (METH == M_WL) {
+        w.wl_gamma = wl_gamma;
+        w.wl_num_states = wl_Ns;
+        w.wl_min_energy = wl_min_e;
+        w.wl_lowest_hist = wl_lowest;
+        w.wl_highest_hist = wl_highest;
+        w.wl_total_hist = wl_total;
+        w.wl_len = wl_len;
+      }
+    }
+    store_common(walker);
+  }
+  SADMC_DF void store_common(int walker) {
     if (lane == 0) {
       sadmc_walker_state &w = args().ws[walker];
       w.rng[0] = s0;
       w.rng[1] = s1;
       w.E = E;
       w.error = err;
-      w.moves = moves;
+      w.moves = moves();
       w.accepted_moves = accepted;
       w.acceptance_rate = acc_rate;
       w.translation_scale = tscale;
@@ -320,28 +342,6 @@ struct Engine {
       w.bulk_visited = (uint64_t)bulk;
       w.status = status;
       w.method = method;
-      if (all || METH == M_SAD) {
-        w.too_lo = too_lo;
-        w.too_hi = too_hi;
-        w.latest_parameter = lam;
-        w.min_T = min_T;
-        w.tL = tL;
-        w.tF = tF;
-        w.num_states = Ns;
-        w.highest_hist = highest;
-        w.tmax = tmax;
-      }
-      if (all || METH == M_SAMC || METH == M_WL) w.t0 = t0;
-      if (all || METH == M_WL) {
-        w.wl_gamma = wl_gamma;
-        w.wl_num_states = wl_Ns;
-        w.wl_min_energy = wl_min_e;
-        w.wl_lowest_hist = wl_lowest;
-        w.wl_highest_hist = wl_highest;
-        w.wl_total_hist = wl_total;
-        w.wl_len = wl_len;
-      }
-      if (all || SYS == SYS_WCA) w.has_pressure = has_pressure;
       if (status) *args().flag = 1;
     }
     if (SYS == SYS_ISING) {
@@ -364,14 +364,16 @@ struct Engine {
   // Bins::state_to_index (energy.rs:371-373); `as usize` saturates.
   // The quotient by the width is first formed with the reciprocal; only
   // when that lands within 1e-9 of an integer (where the two roundings could
-  // truncate differently) is the division itself computed.
+  // truncate differently) or outside (0, 1e6) is the division itself computed.
   SADMC_DF int32_t e_index(double e) const {
     const double d = e - bmin;
-    double v = d * args().inv_width;
-    const double f = v - trunc(v);
-    if (!(f > 1e-9 && f < 1.0 - 1e-9 && v < 1.0e6)) v = d / args().width;
-    if (!(v > 0.0)) return 0;
-    if (v >= 2.0e9) return 0x7fffffff;
+    const double v = d * args().inv_width;
+    if (__builtin_expect(!(fabs(__builtin_amdgcn_fract(v) - 0.5) < 0.5 - 1e-9 && fabs(v - 5.0e5) < 5.0e5), 0)) {
+      const double q = d / args().width;
+      if (!(q > 0.0)) return 0;
+      if (q >= 2.0e9) return 0x7fffffff;
+      return (int32_t)q;
+    }
     return (int32_t)v;
   }
   SADMC_DF double i_energy(int32_t i) const { return bmin + ((double)i + 0.5) * args().width; }
@@ -386,44 +388,37 @@ struct Engine {
   SADMC_DF uint64_t hist_at(int32_t p) const { return p == cur_p ? c_hist : H[p].hist; }
   SADMC_DF uint64_t wlh_at(int32_t p) const { return p == cur_p ? c_wlh : WH[p]; }
 
-  // Cold record of the current bin: written back when the walker leaves the
-  // bin, loaded for the new bin, and first used one move later.
-  SADMC_DF void write_cold() {
-    if (kp >= 0) {
-      Cb[kp].etot = k_etot;
-      Cb[kp].esq = k_esq;
-      Cb[kp].rt = k_rt;
-      Cb[kp].vep = k_vep;
+  // The current bin's record goes back to memory when the walker leaves the
+  // bin or the launch ends (every read in between takes the registers).
+  SADMC_DF void write_back() {
+    if (cur_p >= 0) {
+      HotBin hb;
+      hb.lnw = c_lnw;
+      hb.hist = c_hist;
+      H[cur_p] = hb;
+      ColdBin cb;
+      cb.etot = c_etot;
+      cb.esq = c_esq;
+      cb.rt = c_rt;
+      cb.vep = c_vep;
+      Cb[cur_p] = cb;
     }
   }
-  SADMC_DF void switch_cold(int32_t p) {
-    write_cold();
-    const ColdBin &q = Cb[p];
-    k_etot = q.etot;
-    k_esq = q.esq;
-    k_rt = q.rt;
-    k_vep = q.vep;
-    kp = p;
-  }
-  // energy.rs:941-943 and 950-965 for the previous move: the energy sums and,
-  // when the round-trip branch reached have_visited, its test and update.
-  SADMC_DF void apply_pending() {
-    if (pend) {
-      k_etot += pend_E;
-      k_esq += pend_E * pend_E;
-      if (pend_rt && !(pend_bulk || k_vep == pend_epoch)) {
-        k_vep = pend_epoch;
-        k_rt += 1;
-      }
-      pend = 0;
-    }
-  }
-  SADMC_DF void set_current(int32_t p, double lnw, uint64_t hist) {
-    c_lnw = lnw;
-    c_hist = hist;
-    if (METH == M_WL) c_wlh = WH[p];
+  SADMC_DF void set_current(int32_t p, const HotBin &hb, const ColdBin &cb, uint64_t wlh) {
+    write_back();
     cur_p = p;
-    switch_cold(p);
+    c_lnw = hb.lnw;
+    c_hist = hb.hist;
+    if (METH == M_WL) c_wlh = wlh;
+    c_etot = cb.etot;
+    c_esq = cb.esq;
+    c_rt = cb.rt;
+    c_vep = cb.vep;
+  }
+  SADMC_DF void load_current(int32_t p) {
+    const HotBin hb = H[p];
+    const ColdBin cb = Cb[p];
+    set_current(p, hb, cb, METH == M_WL ? WH[p] : 0);
   }
 
   // Re-derive every cached index from its inputs (after init, resume or a
@@ -435,17 +430,14 @@ struct Engine {
     cur_i = i;
     if (i < len) {
       int32_t p = base + i;
-      if (p != cur_p) {
-        HotBin hb = H[p];
-        set_current(p, hb.lnw, hb.hist);
-      }
+      if (p != cur_p) load_current(p);
     } else {
+      write_back();
       cur_p = -1;
     }
     if (METH == M_SAD) {
       ilo = e_index(too_lo);
       ihi = e_index(too_hi);
-      lnw_lo = ilo < len ? lnw_at(base + ilo) : 0.0;
       lnw_hi = ihi < len ? lnw_at(base + ihi) : 0.0;
     }
   }
@@ -460,10 +452,10 @@ struct Engine {
   SADMC_DF void reset_checks() {
     if (SYS != SYS_ISING) {
       uint64_t P = args().refresh > 0 ? (uint64_t)args().refresh : (uint64_t)len * (uint64_t)len * 1000ULL;
-      next_check = (moves / P + 1) * P;
+      next_check = (double)((moves() / P + 1) * P);
       if (SYS == SYS_WCA) {
         uint64_t Q = (uint64_t)n * (uint64_t)n;
-        next_press = (moves / Q + 1) * Q;
+        next_press = (double)((moves() / Q + 1) * Q);
       }
     }
   }
@@ -471,37 +463,38 @@ struct Engine {
   // energy.rs:400-434 (prepare_for_state) for every energy in [lo, hi]: the
   // bins grow to both ends.  New slots get have_visited = true (visit_epoch =
   // epoch) and round_trips = 1; every other field is already zero.
-  SADMC_DF bool prepare_for_range(double lo, double hi) {
+  // A window without room stops the walker.
+  SADMC_DF void prepare_for_range(double lo, double hi) {
     bool front = false, grew = false;
-    while (lo < bmin) {
+    while (status == 0 && lo < bmin) {
       if (base == 0) {
         status = SADMC_WS_CAPACITY;
-        return false;
+      } else {
+        base -= 1;
+        len += 1;
+        Cb[base].rt = 1;
+        Cb[base].vep = epoch;
+        bmin -= args().width;
+        front = true;
       }
-      base -= 1;
-      len += 1;
-      Cb[base].rt = 1;
-      Cb[base].vep = epoch;
-      bmin -= args().width;
-      front = true;
     }
-    while (hi >= bmin + args().width * (double)len) {
-      int32_t q = base + len;
+    while (status == 0 && hi >= bmin + args().width * (double)len) {
+      const int32_t q = base + len;
       if (q >= args().cap) {
         status = SADMC_WS_CAPACITY;
-        return false;
+      } else {
+        Cb[q].rt = 1;
+        Cb[q].vep = epoch;
+        len += 1;
+        grew = true;
       }
-      Cb[q].rt = 1;
-      Cb[q].vep = epoch;
-      len += 1;
-      grew = true;
     }
-    if (front || (grew && !indices_valid())) refresh_indices();
-    if ((front || grew) && SYS != SYS_ISING && args().refresh <= 0) {
+    btop = bmin + args().width * (double)len;
+    if (status == 0 && (front || (grew && !indices_valid()))) refresh_indices();
+    if (status == 0 && (front || grew) && SYS != SYS_ISING && args().refresh <= 0) {
       uint64_t P = (uint64_t)len * (uint64_t)len * 1000ULL;
-      next_check = (moves / P + 1) * P;
+      next_check = (double)((moves() / P + 1) * P);
     }
-    return status == 0;
   }
 
   // ------------------------------------------------------------ systems
@@ -522,21 +515,19 @@ struct Engine {
         }
       return e;
     }
+    // rare: one small loop from the LDS mirror instead of KMAX unrolled ones
     double acc = 0.0;
-#pragma unroll
-    for (int k = 0; k < KMAX; k++) {
-      if (k < K) {
-        int i = lane + G * k;
-        if (i < n) {
-          for (int j = 0; j < i; j++) {
-            if (SYS == SYS_LJ) {
-              acc += lj_pair(norm2(xk(k) - lx[j], yk(k) - ly[j], zk(k) - lz[j]));
-            } else {
-              acc += wca_pair(norm2(min_image(xk(k) - lx[j], L, halfL), min_image(yk(k) - ly[j], L, halfL),
-                                    min_image(zk(k) - lz[j], L, halfL)),
-                              args().rc2);
-            }
-          }
+#pragma unroll 1
+    for (int i = lane; i < n; i += G) {
+      const double xi = lx[i], yi = ly[i], zi = lz[i];
+#pragma unroll 1
+      for (int j = 0; j < i; j++) {
+        if (SYS == SYS_LJ) {
+          acc += lj_pair(norm2(xi - lx[j], yi - ly[j], zi - lz[j]));
+        } else {
+          acc += wca_pair(norm2(min_image(xi - lx[j], L, halfL), min_image(yi - ly[j], L, halfL),
+                                min_image(zi - lz[j], L, halfL)),
+                          args().rc2);
         }
       }
     }
@@ -546,18 +537,15 @@ struct Engine {
   // wca.rs:202-218 virial, ordered pairs, lane-group order.
   SADMC_DF double pressure() {
     double acc = 0.0;
-#pragma unroll
-    for (int k = 0; k < KMAX; k++) {
-      if (k < K) {
-        int i = lane + G * k;
-        if (i < n) {
-          for (int j = 0; j < n; j++) {
-            if (j == i) continue;
-            acc += wca_pair_pressure(norm2(min_image(xk(k) - lx[j], L, halfL), min_image(yk(k) - ly[j], L, halfL),
-                                           min_image(zk(k) - lz[j], L, halfL)),
-                                     args().rc2);
-          }
-        }
+#pragma unroll 1
+    for (int i = lane; i < n; i += G) {
+      const double xi = lx[i], yi = ly[i], zi = lz[i];
+#pragma unroll 1
+      for (int j = 0; j < n; j++) {
+        if (j == i) continue;
+        acc += wca_pair_pressure(norm2(min_image(xi - lx[j], L, halfL), min_image(yi - ly[j], L, halfL),
+                                       min_image(zi - lz[j], L, halfL)),
+                                 args().rc2);
       }
     }
     double p = group_sum(acc, G);
@@ -567,8 +555,8 @@ struct Engine {
   // ising.rs:104-119.
   SADMC_DF bool ising_plan(double &e2) {
     const int N = n;
-    int i = (int)sample_zone(s0, s1, (uint64_t)N, args().zone_site);
-    int j = (int)sample_zone(s0, s1, (uint64_t)N, args().zone_site);
+    int i = (int)sample_zone(s0, s1, (uint32_t)N, args().zone_site);
+    int j = (int)sample_zone(s0, s1, (uint32_t)N, args().zone_site);
     int jp = j + 1 == N ? 0 : j + 1;
     int jm = j == 0 ? N - 1 : j - 1;
     int ip = i + 1 == N ? 0 : i + 1;
@@ -585,41 +573,35 @@ struct Engine {
   // Uniform::new(-d, d) scale sc); lj.rs:86-105 and wca.rs:119-140 for the
   // energy difference.
   SADMC_DF bool particle_plan(double d, double sc, double &e2) {
-    int w = (int)sample_zone(s0, s1, (uint64_t)n, args().zone_n);
+    int w = (int)sample_zone(s0, s1, (uint32_t)n, args().zone_n);
     double ux = uniform_sample(s0, s1, -d, sc);
     double uy = uniform_sample(s0, s1, -d, sc);
     double uz = uniform_sample(s0, s1, -d, sc);
     double fx = lx[w], fy = ly[w], fz = lz[w];
     double tx, ty, tz;
+    // a move past the wall still runs through the sums below: its wave does
+    // so anyway while any of its walkers moves inside
+    bool some = true;
     if (SYS == SYS_LJ) {
       tx = fx + ux;
       ty = fy + uy;
       tz = fz + uz;
       double r2to = norm2(tx, ty, tz), r2from = norm2(fx, fy, fz);
-      if (r2to > R2 && r2to > r2from) return false;
+      some = !(r2to > R2 && r2to > r2from);
     } else {
       tx = put_in_cell(fx + ux, L);
       ty = put_in_cell(fy + uy, L);
       tz = put_in_cell(fz + uz, L);
     }
-    // Every slot computes its pair terms; the moved atom's own slot and the
-    // padding slots (whose terms may be inf or NaN) are dropped by a select
-    // of the accumulator, which keeps the sums those of the skipped form
-    // without a divergent branch per atom.
     double acc = 0.0, accabs = 0.0;
+    if (SYS == SYS_LJ) {
+      acc = lj_lane_diff(w, tx, ty, tz, fx, fy, fz);
+    } else {
 #pragma unroll
-    for (int k = 0; k < KMAX; k++) {
-      if (k < K) {
-        const int j = lane + G * k;
-        const bool use = j < n && j != w;
-        if (SYS == SYS_LJ) {
-          if (PREC == 0) {
-            const double t = lj_pair(norm2(xk(k) - tx, yk(k) - ty, zk(k) - tz)) -
-                             lj_pair(norm2(xk(k) - fx, yk(k) - fy, zk(k) - fz));
-            const double na = acc + t;
-            acc = use ? na : acc;
-          }
-        } else {
+      for (int k = 0; k < KMAX; k++) {
+        if (k < K) {
+          const int j = lane + G * k;
+          const bool use = j < n && j != w;
           double vn = wca_pair(norm2(min_image(xk(k) - tx, L, halfL), min_image(yk(k) - ty, L, halfL),
                                      min_image(zk(k) - tz, L, halfL)),
                                args().rc2);
@@ -632,7 +614,6 @@ struct Engine {
         }
       }
     }
-    if (SYS == SYS_LJ && PREC == 1) acc = lj32_lane_diff(w, tx, ty, tz, fx, fy, fz);
     double e = E + group_sum(acc, G);
     if (SYS == SYS_WCA) pdabse = group_sum(accabs, G);
     pw = w;
@@ -641,7 +622,7 @@ struct Engine {
     ptz = tz;
     pe = e;
     e2 = e;
-    return true;
+    return some;
   }
 
   // Features of the group's atoms around (px, py, pz), skipping atom w;
@@ -661,65 +642,78 @@ struct Engine {
     for (int c = 0; c < kPropNF; c++) f[c] = group_sum_f32(f[c], G);
   }
 
-  // This lane's sum of the binary32 pair-term differences V(|x_j - t|^2) -
-  // V(|x_j - f|^2) over its atoms j != w (lj.rs:86-105 in FP32 pair terms,
-  // accumulated in FP64), 1/r^2 from recip_f32_fast when FAST, else from the
-  // division.
-  template <bool FAST>
-  SADMC_DF double lj32_lane_sum(int w, double tx, double ty, double tz, double fx, double fy, double fz) {
+  // This lane's sum of the pair-term differences V(|x_j - t|^2) -
+  // V(|x_j - f|^2) over its atoms j != w (lj.rs:86-105; in the precision
+  // variant binary32 terms accumulated in FP64), with the fast reciprocals.
+  // Every slot computes its terms; the moved atom's own slot and the padding
+  // slots (whose terms may be inf or NaN) are dropped by a select of the
+  // accumulator, which keeps the sums those of the skipped form without a
+  // divergent branch per atom.
+  SADMC_DF double lj_lane_sum(int w, double tx, double ty, double tz, double fx, double fy, double fz) {
     double acc = 0.0;
 #pragma unroll
     for (int k = 0; k < KMAX; k++) {
       if (k < K) {
         const int j = lane + G * k;
         const bool use = j < n && j != w;
-        const float an = (float)(xk(k) - tx), bn = (float)(yk(k) - ty), cn = (float)(zk(k) - tz);
-        const float ao = (float)(xk(k) - fx), bo = (float)(yk(k) - fy), co = (float)(zk(k) - fz);
-        const float r2n = an * an + bn * bn + cn * cn;
-        const float r2o = ao * ao + bo * bo + co * co;
-        const double t = FAST ? (double)lj_pair_f32_fast(r2n) - (double)lj_pair_f32_fast(r2o)
-                              : (double)lj_pair_f32(r2n) - (double)lj_pair_f32(r2o);
+        double t;
+        if (PREC == 1) {
+          const float an = (float)(xk(k) - tx), bn = (float)(yk(k) - ty), cn = (float)(zk(k) - tz);
+          const float ao = (float)(xk(k) - fx), bo = (float)(yk(k) - fy), co = (float)(zk(k) - fz);
+          t = (double)lj_pair_f32_fast(an * an + bn * bn + cn * cn) -
+              (double)lj_pair_f32_fast(ao * ao + bo * bo + co * co);
+        } else {
+          t = lj_pair_fast(norm2(xk(k) - tx, yk(k) - ty, zk(k) - tz)) -
+              lj_pair_fast(norm2(xk(k) - fx, yk(k) - fy, zk(k) - fz));
+        }
         const double na = acc + t;
         acc = use ? na : acc;
       }
     }
     return acc;
   }
+  // The same with the divisions; hardly ever needed, so a small loop over the
+  // LDS mirror.
+  SADMC_DF double lj_lane_sum_div(int w, double tx, double ty, double tz, double fx, double fy, double fz) {
+    double acc = 0.0;
+#pragma unroll 1
+    for (int j = lane; j < n; j += G) {
+      if (j == w) continue;
+      const double xj = lx[j], yj = ly[j], zj = lz[j];
+      if (PREC == 1) {
+        const float an = (float)(xj - tx), bn = (float)(yj - ty), cn = (float)(zj - tz);
+        const float ao = (float)(xj - fx), bo = (float)(yj - fy), co = (float)(zj - fz);
+        acc += (double)lj_pair_f32(an * an + bn * bn + cn * cn) - (double)lj_pair_f32(ao * ao + bo * bo + co * co);
+      } else {
+        acc += lj_pair(norm2(xj - tx, yj - ty, zj - tz)) - lj_pair(norm2(xj - fx, yj - fy, zj - fz));
+      }
+    }
+    return acc;
+  }
 
-  // lj32_lane_sum with the fast reciprocal, equal to the division's sum bit
-  // for bit: the two reciprocals agree on [2^-126, 2^126); below 2^-126
-  // 1/r^2 exceeds 2^126, so s^6 overflows and the pair term is NaN with
-  // either; from 2^126 up s^2 underflows and both terms are +0; at +inf
-  // only the fast one is NaN.  So the fast sum differs only where it is
-  // NaN, and then the lanes still running this code recompute with the
-  // division.
-  SADMC_DF double lj32_lane_diff(int w, double tx, double ty, double tz, double fx, double fy, double fz) {
-    double acc = lj32_lane_sum<true>(w, tx, ty, tz, fx, fy, fz);
-    if (__builtin_expect(__any(acc != acc), 0)) acc = lj32_lane_sum<false>(w, tx, ty, tz, fx, fy, fz);
+  // lj_lane_sum with the fast reciprocals, equal to the divisions' sum bit
+  // for bit.  Binary32: the two reciprocals agree on [2^-126, 2^126); below
+  // 2^-126 1/r^2 exceeds 2^126, so s^6 overflows and the pair term is NaN
+  // with either; from 2^126 up s^2 underflows and both terms are +0; at +inf
+  // only the fast one is NaN.  Binary64: see recip_f64_fast.  So the fast sum
+  // differs only where it is NaN, and then the lanes still running this code
+  // recompute with the division.
+  SADMC_DF double lj_lane_diff(int w, double tx, double ty, double tz, double fx, double fy, double fz) {
+    double acc = lj_lane_sum(w, tx, ty, tz, fx, fy, fz);
+    if (__builtin_expect(__any(acc != acc), 0)) acc = lj_lane_sum_div(w, tx, ty, tz, fx, fy, fz);
     return acc;
   }
 
   // Sum over the group of the pair-term differences for atom w moving from
   // f to t (lj.rs:86-105).
   SADMC_DF double lj_delta(int w, double tx, double ty, double tz, double fx, double fy, double fz) {
-    if (PREC == 1) return group_sum(lj32_lane_diff(w, tx, ty, tz, fx, fy, fz), G);
-    double acc = 0.0;
-#pragma unroll
-    for (int k = 0; k < KMAX; k++) {
-      if (k < K) {
-        int j = lane + G * k;
-        if (j < n && j != w)
-          acc += lj_pair(norm2(xk(k) - tx, yk(k) - ty, zk(k) - tz)) -
-                 lj_pair(norm2(xk(k) - fx, yk(k) - fy, zk(k) - fz));
-      }
-    }
-    return group_sum(acc, G);
+    return group_sum(lj_lane_diff(w, tx, ty, tz, fx, fy, fz), G);
   }
 
   // The learned move: sigma from the network at the old position, a
   // Gaussian step, sigma' at the new position for the Hastings term.
   SADMC_DF bool learned_plan(double &e2) {
-    int w = (int)sample_zone(s0, s1, (uint64_t)n, args().zone_n);
+    int w = (int)sample_zone(s0, s1, (uint32_t)n, args().zone_n);
     const double fx = lx[w], fy = ly[w], fz = lz[w];
     float f[kPropNF], xi[3];
     features(fx, fy, fz, w, f);
@@ -751,7 +745,7 @@ struct Engine {
   SADMC_DF bool sad_lnw(double e, double &out) {
     if (ilo < 0 || ilo >= len || ihi < 0 || ihi >= len) return false;
     if (e < too_lo) {
-      out = lnw_lo + (e - too_lo) / min_T;
+      out = lnw_at(base + ilo) + (e - too_lo) / rec().min_T;
       return true;
     }
     if (e > too_hi) {
@@ -875,19 +869,37 @@ struct Engine {
     }
   }
 
-  // lj.rs:249-261, wca.rs:237-250.
-  SADMC_DF void verify_energy() {
-    double egood = full_energy();
+  // lj.rs:249-261, wca.rs:237-250; `egood` is the recomputed energy.
+  SADMC_DF void verify_energy() { verify_energy(full_energy()); }
+  SADMC_DF void verify_energy(double egood) {
     double nn = (double)n;
     double expected = SYS == SYS_LJ ? fabs(E) * 1e-14 * nn * nn : fabs(E) * 1e-13 * nn * nn;
     if (fabs(egood - E) > expected) status = SADMC_WS_VERIFY;
   }
 
   // ------------------------------------------------------------- method
-  // energy.rs:22-38 with t = moves, tF, N_s (energy.rs:799-813).
+  // energy.rs:22-38 with t = moves, tF, N_s (energy.rs:799-813).  t / tF and
+  // t / N_s come from the kept correctly rounded reciprocals y = RN(1/b):
+  // RN(t y) is within two units of the quotient, the first residual step
+  // brings it to a faithful one, and with a faithful quotient the second
+  // gives the correctly rounded one (Markstein 1990), which is the division's.
+  // The operands are whole numbers below 2^53 (b >= 1; otherwise gamma is 0),
+  // so nothing over- or underflows.
+  SADMC_DF static double quot(double a, double b, double y) {
+    double q = a * y;
+    q = __builtin_fma(__builtin_fma(-b, q, a), y, q);
+    return __builtin_fma(__builtin_fma(-b, q, a), y, q);
+  }
   SADMC_DF double sad_gamma() const {
-    if (lam * tF_d * Ns_d == 0.0) return 0.0;
-    return (lam + tm / tF_d) / (lam + tm / Ns_d * (tm / tF_d));
+    const double q = quot(tm, tF, rtF);
+    const double g = (lam + q) / (lam + quot(tm, Ns, rNs) * q);
+    return gzero ? 0.0 : g;
+  }
+  // After a change of lam, tF or Ns.
+  SADMC_DF void gamma_changed() {
+    rtF = 1.0 / tF;
+    rNs = 1.0 / Ns;
+    gzero = lam * tF * Ns == 0.0;
   }
 
   // Draw the next uniform ahead of the test that may use it.
@@ -903,78 +915,76 @@ struct Engine {
   // rounds to float with |dt| <= |t| 2^-24, v_exp_f32 is within a few ulp
   // (2^-21), so the estimate is within |t| 2^-24 ln 2 + 2^-21 < 1e-7 |t| +
   // 1e-6 of exp(x), and of the correctly rounded double exp (2^-53 more);
-  // the band is ten times that.  Below t = -125 exp(x) < 2^-125 lies under
-  // every nonzero u (multiples of 2^-53), so the test is u > 0.  NaN and
-  // x >= 0 take the double path.
+  // the band is ten times that.  Below t = -125 exp(x) < 2^-125 and the
+  // estimate (possibly flushed to 0) lie under every nonzero u (multiples of
+  // 2^-53); u = 0 and NaN take the double path.  When `need` holds, x <= 0.
   SADMC_DF bool mh_test(bool need, double x) {
-    if (!need) return false;
-    s0 = spec0;
-    s1 = spec1;
-    const double t = x * 1.4426950408889634;
-    if (t < -125.0) return spec_u > 0.0;
-    if (t <= 0.0) {
-      const double est = (double)__builtin_amdgcn_exp2f((float)t);
-      const double band = est * (1e-5 - 1e-6 * t);
-      if (spec_u > est + band) return true;
-      if (spec_u < est - band) return false;
-    }
-    return spec_u > exp(x);
+    s0 = need ? spec0 : s0;
+    s1 = need ? spec1 : s1;
+    double t = x * 1.4426950408889634;
+    t = t < -1000.0 ? -1000.0 : t;  // the estimate is 0 from there on, and -inf would make the band NaN
+    const double est = (double)__builtin_amdgcn_exp2f((float)t);
+    const double band = est * (1e-5 - 1e-6 * t);
+    bool rejected = spec_u > est + band;
+    if (__builtin_expect(need && !rejected && !(spec_u < est - band), 0)) rejected = spec_u > exp(x);
+    return need && rejected;
   }
   // Metropolis-Hastings test on the log acceptance ratio.
-  SADMC_DF bool reject_lr(double lr) { return mh_test(lr < 0.0, lr); }
+  SADMC_DF bool reject_lr(bool go, double lr) { return mh_test(go && lr < 0.0, lr); }
   // ln w(e) with the SAD clamped extension (energy.rs:445-463); `inside` is
   // the bin's ln w.
   SADMC_DF double sad_lnw_ext(double e, double inside) const {
-    if (e < too_lo) return lnw_lo + (e - too_lo) / min_T;
-    if (e > too_hi) return lnw_hi;
-    return inside;
+    double v = e > too_hi ? lnw_hi : inside;
+    if (__builtin_expect(e < too_lo, 0)) v = lnw_at(base + ilo) + (e - too_lo) / rec().min_T;
+    return v;
   }
 
-  // energy.rs:440-512.  `r2` is the record of the proposed bin.  The
+  // energy.rs:440-512.  `r2` is the record of the proposed bin; nothing
+  // happens for a walker without a move to test (`go` false).  The
   // learned move adds ln H to the exponent (the tests are the reference's
   // when ln H = 0).
-  SADMC_DF bool reject_move(double e1, double e2, double r2_lnw, uint64_t r2_hist) {
+  SADMC_DF bool reject_move(bool go, double e1, double e2, double r2_lnw, uint64_t r2_hist) {
     if (MV == 1) {
       if (METH == M_SAD) {
         const double lnw1 = sad_lnw_ext(e1, c_lnw), lnw2 = sad_lnw_ext(e2, r2_lnw);
-        bool rejected = reject_lr(lnw1 - lnw2 + lnh);
-        if (!rejected && r2_hist == 0 && e2 < too_hi && e2 > too_lo) {
-          lam = (too_hi - too_lo) / min_T;
-          Ns += 1;
-          Ns_d = (double)Ns;
-          tL = moves;
-          gdirty = true;
+        bool rejected = reject_lr(go, lnw1 - lnw2 + lnh);
+        if (__builtin_expect(go && !rejected && r2_hist == 0, 0) && e2 < too_hi && e2 > too_lo) {
+          lam = (too_hi - too_lo) / rec().min_T;
+          Ns += 1.0;
+          set_tL();
+          gamma_changed();
+          gpre = sad_gamma();
         }
         return rejected;
       } else if (METH == M_SAMC) {
-        return reject_lr(c_lnw - r2_lnw + lnh);
+        return reject_lr(go, c_lnw - r2_lnw + lnh);
       } else if (METH == M_WL) {
-        bool rejected = reject_lr(c_lnw - r2_lnw + lnh);
-        if (method != SADMC_SAMC && !rejected && r2_hist == 0 && wl_lowest > 0) wl_Ns += 1.0;
+        bool rejected = reject_lr(go, c_lnw - r2_lnw + lnh);
+        if (go && method != SADMC_SAMC && !rejected && r2_hist == 0 && wl_lowest > 0) wl_Ns += 1.0;
         return rejected;
       } else {
-        return reject_lr((e1 - e2) / args().method_param + lnh);
+        return reject_lr(go, (e1 - e2) / args().method_param + lnh);
       }
     }
     if (METH == M_SAD) {
       const double lnw1 = sad_lnw_ext(e1, c_lnw), lnw2 = sad_lnw_ext(e2, r2_lnw);
-      bool rejected = mh_test(lnw2 > lnw1, lnw1 - lnw2);
-      if (!rejected && r2_hist == 0 && e2 < too_hi && e2 > too_lo) {
-        lam = (too_hi - too_lo) / min_T;
-        Ns += 1;
-        Ns_d = (double)Ns;
-        tL = moves;
-        gdirty = true;
+      bool rejected = mh_test(go && lnw2 > lnw1, lnw1 - lnw2);
+      if (__builtin_expect(go && !rejected && r2_hist == 0, 0) && e2 < too_hi && e2 > too_lo) {
+        lam = (too_hi - too_lo) / rec().min_T;
+        Ns += 1.0;
+        set_tL();
+        gamma_changed();
+        gpre = sad_gamma();
       }
       return rejected;
     } else if (METH == M_SAMC) {
-      return mh_test(r2_lnw > c_lnw, c_lnw - r2_lnw);
+      return mh_test(go && r2_lnw > c_lnw, c_lnw - r2_lnw);
     } else if (METH == M_WL) {
-      bool rejected = mh_test(r2_lnw > c_lnw, c_lnw - r2_lnw);
-      if (method != SADMC_SAMC && !rejected && r2_hist == 0 && wl_lowest > 0) wl_Ns += 1.0;
+      bool rejected = mh_test(go && r2_lnw > c_lnw, c_lnw - r2_lnw);
+      if (go && method != SADMC_SAMC && !rejected && r2_hist == 0 && wl_lowest > 0) wl_Ns += 1.0;
       return rejected;
     } else {
-      return mh_test(e1 < e2, (e1 - e2) / args().method_param);
+      return mh_test(go && e1 < e2, (e1 - e2) / args().method_param);
     }
   }
 
@@ -994,41 +1004,43 @@ struct Engine {
     for (int d = 1; d < G; d <<= 1) v += __shfl_xor(v, d, 64);
     return v;
   }
+  SADMC_DF void set_tL() {
+    tl_now = true;
+    rec().tL = moves();
+  }
   SADMC_DF void tmax_scan(int32_t a, int32_t b) {
+    const uint64_t *TF = tfound();
     uint64_t m = 0;
     for (int32_t j = a + lane; j <= b; j += G) {
-      const uint64_t t = Cb[base + j].tfound;
+      const uint64_t t = TF[base + j];
       m = t > m ? t : m;
     }
     m = group_max_u64(m);
-    if (m > tmax) tmax = m;
-  }
-
-  SADMC_DF void set_lnw(int32_t p, double v) {
-    H[p].lnw = v;
-    if (p == cur_p) c_lnw = v;
+    if (m > rec().tmax) rec().tmax = m;
   }
 
   // energy.rs:514-636 for the current bin (logical i = cur_i).
   SADMC_DF void update_sad(double E_, int32_t i) {
     const double E = E_;
     if (!(too_lo > too_hi || E < too_lo || E > too_hi)) {
-      c_lnw += gdirty ? sad_gamma() : gpre;
-      if (cur_p == base + ilo) lnw_lo = c_lnw;
+      c_lnw += gpre;
       if (cur_p == base + ihi) lnw_hi = c_lnw;
     }
+    if (__builtin_expect(c_hist > highest || tl_now, 0)) update_sad_range(E, i);
+  }
+  // The part of update_sad that a new highest count or a new tL needs.
+  SADMC_DF void update_sad_range(double E, int32_t i) {
     if (c_hist > highest) {
       highest = c_hist;
-      // the cached ln w at too_lo / too_hi and N_s change here only when
-      // the range grows; otherwise ln w at those bins changes only through
-      // the current bin, which the increment above already tracks
+      // the cached ln w at too_hi and N_s change here only when the range
+      // grows; otherwise ln w at that bin changes only through the current
+      // bin, which the increment above already tracks
       bool grew = false;
-      if (E > too_hi) {
+      const double min_T = rec().min_T;
+      if ((E > too_hi && ihi >= len) || (E < too_lo && ilo >= len)) {
+        status = SADMC_WS_INDEX;
+      } else if (E > too_hi) {
         grew = true;
-        if (ihi >= len) {
-          status = SADMC_WS_INDEX;
-          return;
-        }
         const double vhi = lnw_hi;
         int32_t jlo = ihi > 0 ? ihi - 1 : 0, jhi = i + 1 < len ? i + 1 : len - 1;
         uint32_t cnt = 0;
@@ -1049,30 +1061,22 @@ struct Engine {
             cnt += c_hist != 0 ? 1u : 0u;
           }
         }
-        Ns += cnt;
+        Ns += (double)cnt;
         __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
         lam = (E - too_lo) / min_T;
-        tL = moves;
+        set_tL();
         double nh = i_energy(i);
         int32_t ihi2 = e_index(nh);
         if (ihi2 > ihi) tmax_scan(ihi + 1, ihi2 < len ? ihi2 : len - 1);
         too_hi = nh;
         ihi = ihi2;
-        if (ihi >= len) {
-          status = SADMC_WS_INDEX;
-          return;
-        }
+        if (ihi >= len) status = SADMC_WS_INDEX;
       } else if (E < too_lo) {
         grew = true;
-        if (ilo >= len) {
-          status = SADMC_WS_INDEX;
-          return;
-        }
         // every bin below too_lo extends from the old ln w(too_lo): the bin
-        // of too_lo itself comes last in energy order, and ln w(too_lo) is
-        // reloaded from the new range below
+        // of too_lo itself comes last in energy order
         int32_t jlo = i > 0 ? i - 1 : 0, jhi = ilo + 1 < len ? ilo + 1 : len - 1;
-        const double vlo = lnw_lo;
+        const double vlo = lnw_at(base + ilo);
         uint32_t cnt = 0;
         for (int32_t j = jlo + lane; j <= jhi; j += G) {
           const double ej = i_energy(j);
@@ -1101,30 +1105,22 @@ struct Engine {
             cnt += c_hist != 0 ? 1u : 0u;
           }
         }
-        Ns += cnt;
+        Ns += (double)cnt;
         __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
         lam = (too_hi - E) / min_T;
-        tL = moves;
+        set_tL();
         double nl = i_energy(i);
         int32_t ilo2 = e_index(nl);
         if (ilo2 < ilo) tmax_scan(ilo2, ilo - 1);
         too_lo = nl;
         ilo = ilo2;
       }
-      if (grew) {
-        Ns_d = (double)Ns;
-        lnw_lo = lnw_at(base + ilo);
-        lnw_hi = lnw_at(base + ihi);
-      }
+      if (grew && status == 0) lnw_hi = lnw_at(base + ihi);
     }
-    if (tL == moves) {
-      if (ilo >= len || ihi >= len) {
-        status = SADMC_WS_INDEX;
-        return;
-      }
-      uint64_t old_tF = tF;
-      tF = tmax;
-      tF_d = (double)tF;
+    if (tl_now && status == 0 && (ilo >= len || ihi >= len)) status = SADMC_WS_INDEX;
+    if (tl_now && status == 0) {
+      const double old_tF = tF;
+      tF = (double)rec().tmax;
       if (old_tF != tF && args().move_plan == SADMC_ACCEPTANCE_RATE) {
         double s = acc_rate / args().move_param;
         s = s < 0.8 ? 0.8 : (s > 1.2 ? 1.2 : s);
@@ -1132,6 +1128,7 @@ struct Engine {
         if (SYS != SYS_ISING) usc = uniform_scale(-tscale, tscale);
       }
     }
+    gamma_changed();
   }
 
   // energy.rs:638-756 (WL and 1/t-WL); SAMC after the 1/t switch.
@@ -1216,31 +1213,34 @@ struct Engine {
     }
   }
 
-  // energy.rs:904-974.
+  // energy.rs:904-974.  One memory round trip per move: both parts of the
+  // proposed bin's record are requested as soon as its energy is known, for
+  // every lane (a walker whose proposal is void reads its current bin), and
+  // what does not need them is computed meanwhile.  What is common is written
+  // as selects rather than branches, which the walkers of a wave would
+  // otherwise take one after the other; the rare parts stay branches.
   SADMC_DF void move_once() {
     bool regrow = false;
-    moves += 1;
     tm += 1.0;
-    gdirty = true;
-    if (SYS != SYS_ISING && moves == next_check) {
+    if (METH == M_SAD) tl_now = false;
+    if (SYS != SYS_ISING && __builtin_expect(tm == next_check, 0)) {
+      const double egood = full_energy();
       if (args().refresh > 0) {
-        E = full_energy();
-        next_check += (uint64_t)args().refresh;
+        E = egood;
+        next_check += (double)args().refresh;
         // the refreshed energy may lie in another bin than the tracked one
         // (move_once indexes the bins by the energy itself, energy.rs:904-974),
         // or past the window's edge by the FP32 drift: the window then grows
         // to it as for a proposed energy (energy.rs:400-434), together with
         // the proposal's growth below (the order of the two growths does not
-        // change the bins they add); the previous move's pending sums belong
-        // to the bin it left
+        // change the bins they add)
         if (e_index(E) != cur_i || E < bmin) {
-          apply_pending();
           refresh_indices();
           regrow = cur_p < 0 || E < bmin;
         }
       } else {
-        verify_energy();
-        next_check += (uint64_t)len * (uint64_t)len * 1000ULL;
+        verify_energy(egood);
+        next_check += (double)((uint64_t)len * (uint64_t)len * 1000ULL);
       }
     }
     const double e1 = E;
@@ -1258,85 +1258,73 @@ struct Engine {
       rs_next += 1;
     }
     acc_rate *= 1.0 - rs;
-    double e2;
-    const bool some = plan_move(tscale, usc, e2);
-    apply_pending();
-    bool go = false;
-    if (some) {
-      bool oob = false;
-      if (args().has_max_e) oob = e2 > args().max_e && e2 > e1;
-      if (args().has_min_e) oob = oob || (e2 < args().min_e && e2 < e1);
-      go = !oob;
-    }
-    if (go || regrow) {
+    double e2 = e1;
+    bool go = plan_move(tscale, usc, e2);
+    if (args().has_max_e) go = go && !(e2 > args().max_e && e2 > e1);
+    if (args().has_min_e) go = go && !(e2 < args().min_e && e2 < e1);
+    if (__builtin_expect(regrow || (go && (e2 < bmin || e2 >= btop)), 0)) {
       double lo = go ? e2 : E, hi = lo;
       if (regrow) {
         lo = E < lo ? E : lo;
         hi = E > hi ? E : hi;
       }
-      if (!prepare_for_range(lo, hi)) return;
+      prepare_for_range(lo, hi);
     }
-    if (go) {
-      i1 = cur_i;
-      int32_t i2 = e_index(e2);
-      if (!indices_valid() || !idx_ok(i2)) {
-        status = SADMC_WS_INDEX;
-        return;
-      }
-      const int32_t p2 = base + i2;
-      double w2;
-      uint64_t h2;
-      if (p2 == cur_p) {
-        w2 = c_lnw;
-        h2 = c_hist;
-      } else {
-        HotBin hb = H[p2];
-        w2 = hb.lnw;
-        h2 = hb.hist;
-      }
-      // independent of the record being loaded
-      if (METH == M_SAD) {
-        gpre = sad_gamma();
-        gdirty = false;
-      }
-      spec_draw();
-      if (!reject_move(e1, e2, w2, h2)) {
-        accepted += 1;
-        acc_rate += rs;
-        confirm();
-        int32_t i = (E == e2) ? i2 : e_index(E);
-        if (!idx_ok(i)) return;
-        const int32_t p = base + i;
-        if (p != cur_p) {
-          if (p == p2) {
-            set_current(p, w2, h2);
-          } else {
-            HotBin hb = H[p];
-            set_current(p, hb.lnw, hb.hist);
-          }
-        }
-        cur_i = i;
-      }
-    }
-    if (status) return;
-    if (cur_p < 0) {
+    i1 = go ? cur_i : i1;
+    const int32_t i2 = go ? e_index(e2) : cur_i;
+    if (status == 0 && (cur_p < 0 || (go && (!indices_valid() || (uint32_t)i2 >= (uint32_t)len))))
       status = SADMC_WS_INDEX;
-      return;
+    if (__builtin_expect(status == 0, 1)) finish_move(go, e1, e2, i1, i2, rs);
+  }
+
+  // The second half of a move: the test, the accepted move's bookkeeping and
+  // the update of the bin the walker is in.
+  SADMC_DF void finish_move(bool go, double e1, double e2, int32_t i1, int32_t i2, double rs) {
+    const int32_t p2 = go ? base + i2 : cur_p;
+    const HotBin hb = H[p2];
+    const ColdBin cb = Cb[p2];
+    uint64_t wl2 = 0;
+    if (METH == M_WL) wl2 = WH[p2];
+    // independent of the record being loaded
+    if (METH == M_SAD) gpre = sad_gamma();
+    spec_draw();
+    const bool same = p2 == cur_p;
+    const double w2 = same ? c_lnw : hb.lnw;
+    const uint64_t h2 = same ? c_hist : hb.hist;
+    const bool acc = !reject_move(go, e1, e2, w2, h2) && go;
+    accepted += acc ? 1 : 0;
+    acc_rate = acc ? acc_rate + rs : acc_rate;
+    if (acc) {
+      confirm();
+      int32_t i = i2;
+      if (__builtin_expect(E != e2, 0)) i = e_index(E);
+      if (__builtin_expect(i != i2, 0)) {
+        if (idx_ok(i) && base + i != cur_p) load_current(base + i);
+      } else if (!same) {
+        set_current(p2, hb, cb, wl2);
+      }
+      cur_i = i;
     }
+    if (__builtin_expect(status == 0, 1)) visit(i1);
+  }
+  SADMC_DF void visit(int32_t i1) {
     const double En = E;
     const int32_t i = cur_i;
     const int32_t p = cur_p;
-    if (c_hist == 0) {
-      Cb[p].tfound = moves;
-      if (METH == M_SAD && i >= ilo && i <= ihi) tmax = moves;
+    if (__builtin_expect(c_hist == 0, 0)) {
+      tfound()[p] = moves();
+      if (METH == M_SAD && i >= ilo && i <= ihi) rec().tmax = moves();
     }
     c_hist += 1;
-    if (SYS == SYS_WCA && args().collect_pressure && moves == next_press) {
-      double pv = pressure();
-      has_pressure = 1;
-      X[p].count += 1;
-      X[p].total += pv;
-      next_press += (uint64_t)n * (uint64_t)n;
+    if (SYS == SYS_WCA && args().collect_pressure && __builtin_expect(tm == next_press, 0)) {
+      const double pv = pressure();
+      PExtra &x = args().extra[(int64_t)wk * args().cap + p];
+      rec().has_pressure = 1;
+      if (lane == 0) {
+        x.count += 1;
+        x.total += pv;
+      }
+      next_press += (double)n * (double)n;
     }
     if (METH == M_SAD) {
       update_sad(En, i);
@@ -1345,38 +1333,38 @@ struct Engine {
     } else if (METH == M_WL) {
       update_wl(i);
     }
-    {
-      HotBin hb;
-      hb.lnw = c_lnw;
-      hb.hist = c_hist;
-      H[p] = hb;
-    }
-    if (status) return;
-    int32_t rt_cand = 0;
-    if (c_lnw > max_S) {
-      max_S = c_lnw;
-      max_S_index = i;
-      epoch += 1;
-      bulk = 1;
-    } else if (i == max_S_index) {
-      if (i1 != i) {
+    if (__builtin_expect(status == 0, 1)) after_visit(En, i, i1);
+  }
+  SADMC_DF void after_visit(double En, int32_t i, int32_t i1) {
+    // energy.rs:950-965 and 941-943 (the energy of this move's end is added
+    // at the start of the next in the reference; nothing between reads it)
+    bool round_trip = true;
+    if (__builtin_expect(c_lnw > max_S || i == max_S_index, 0)) {
+      round_trip = false;
+      if (c_lnw > max_S) {
+        max_S = c_lnw;
+        max_S_index = i;
+        epoch += 1;
+        bulk = 1;
+      } else if (i1 != i) {
         epoch += 1;
         bulk = 0;
       }
-    } else {
-      rt_cand = 1;
     }
-    pend = 1;
-    pend_E = En;
-    pend_rt = rt_cand;
-    pend_epoch = epoch;
-    pend_bulk = bulk;
+    if (round_trip && !(bulk || c_vep == epoch)) {
+      c_vep = epoch;
+      c_rt += 1;
+    }
+    c_etot += En;
+    c_esq += En * En;
   }
 
   SADMC_DF void run(uint64_t nmoves) {
-    for (uint64_t k = 0; k < nmoves; k++) {
-      if (status) break;
-      move_once();
+    // (the loop's exit is the wave's, not a walker's: a divergent exit makes
+    // the compiler keep the state of stopped and running walkers apart, which
+    // took 80 more registers)
+    for (uint64_t k = 0; k < nmoves && __any(status == 0); k++) {
+      if (__builtin_expect(status == 0, 1)) move_once();
     }
   }
 
@@ -1423,37 +1411,42 @@ struct Engine {
       cb.esq = E * E;
       cb.rt = 1;
       cb.vep = 0;
-      cb.tfound = 0;
-      cb.pad = 0;
       Cb[base] = cb;
     }
     max_S = 0.0;
     max_S_index = 0;
     epoch = 1;
     bulk = 0;
-    moves = 0;
+    tm = 0.0;
     accepted = 0;
     acc_rate = 0.5;
     tscale = args().move_plan == SADMC_TRANSLATION_SCALE ? args().move_param : 0.05;
     method = args().method;
-    min_T = args().method == SADMC_SAD ? args().method_param : 0.0;
-    t0 = args().method == SADMC_SAMC ? args().method_param : 0.0;
-    too_lo = E;
-    too_hi = E;
-    tL = 0;
-    tF = 0;
-    Ns = 1;
-    highest = 1;
-    lam = 0.0;
-    tmax = 0;
-    wl_gamma = 1.0;
-    wl_lowest = (args().has_min_e && args().has_max_e) ? 0 : 1;
-    wl_highest = 1;
-    wl_total = 0;
-    wl_Ns = (args().has_min_e && args().has_max_e) ? (args().max_e - args().min_e) / width : 1.0;
-    wl_len = 0;
-    wl_min_e = E;
-    has_pressure = 0;
+    t0 = 0.0;
+    // every method's fields, also those store() leaves to the record
+    if (lane == 0) {
+      sadmc_walker_state &q = rec();
+      q.min_T = args().method == SADMC_SAD ? args().method_param : 0.0;
+      q.t0 = args().method == SADMC_SAMC ? args().method_param : 0.0;
+      q.too_lo = E;
+      q.too_hi = E;
+      q.latest_parameter = 0.0;
+      q.tL = 0;
+      q.tF = 0;
+      q.num_states = 1;
+      q.highest_hist = 1;
+      q.tmax = 0;
+      const bool both = args().has_min_e && args().has_max_e;
+      q.wl_gamma = 1.0;
+      q.wl_lowest_hist = both ? 0 : 1;
+      q.wl_highest_hist = 1;
+      q.wl_total_hist = 0;
+      q.wl_num_states = both ? (args().max_e - args().min_e) / width : 1.0;
+      q.wl_len = 0;
+      q.wl_min_energy = E;
+      q.has_pressure = 0;
+    }
+    store_common(walker);
   }
 };
 

@@ -64,6 +64,7 @@ struct SetHost {
   uint64_t *d_spins = nullptr;
   HotBin *d_hot = nullptr;
   ColdBin *d_cold = nullptr;
+  uint64_t *d_tf = nullptr;
   uint64_t *d_wlh = nullptr;
   PExtra *d_extra = nullptr;
   Pending *d_pending = nullptr;
@@ -289,10 +290,11 @@ static double lj_lowest(int n) {
 static int gather_bins(sadmc_ctx *c, const SetHost &s, int w, int64_t first, int64_t count, sadmc_bin *out) {
   std::vector<HotBin> h(count);
   std::vector<ColdBin> cb(count);
-  std::vector<uint64_t> wl(count, 0);
+  std::vector<uint64_t> tf(count), wl(count, 0);
   const size_t off = (size_t)w * s.cap + first;
   HIPCHECK(c, hipMemcpy(h.data(), s.d_hot + off, sizeof(HotBin) * count, hipMemcpyDeviceToHost));
   HIPCHECK(c, hipMemcpy(cb.data(), s.d_cold + off, sizeof(ColdBin) * count, hipMemcpyDeviceToHost));
+  HIPCHECK(c, hipMemcpy(tf.data(), s.d_tf + off, sizeof(uint64_t) * count, hipMemcpyDeviceToHost));
   if (s.d_wlh) HIPCHECK(c, hipMemcpy(wl.data(), s.d_wlh + off, sizeof(uint64_t) * count, hipMemcpyDeviceToHost));
   for (int64_t k = 0; k < count; k++) {
     out[k].lnw = h[k].lnw;
@@ -301,7 +303,7 @@ static int gather_bins(sadmc_ctx *c, const SetHost &s, int w, int64_t first, int
     out[k].energy_squared_total = cb[k].esq;
     out[k].round_trips = cb[k].rt;
     out[k].visit_epoch = cb[k].vep;
-    out[k].t_found = cb[k].tfound;
+    out[k].t_found = tf[k];
     out[k].wl_hist = wl[k];
   }
   return SADMC_OK;
@@ -373,6 +375,7 @@ static void free_set(SetHost &s) {
   (void)hipFree(s.d_spins);
   (void)hipFree(s.d_hot);
   (void)hipFree(s.d_cold);
+  (void)hipFree(s.d_tf);
   (void)hipFree(s.d_wlh);
   (void)hipFree(s.d_extra);
   (void)hipFree(s.d_pending);
@@ -384,6 +387,7 @@ static void free_set(SetHost &s) {
   s.d_spins = nullptr;
   s.d_hot = nullptr;
   s.d_cold = nullptr;
+  s.d_tf = nullptr;
   s.d_wlh = nullptr;
   s.d_extra = nullptr;
   s.d_pending = nullptr;
@@ -511,6 +515,7 @@ static void fill_args(SetHost &s) {
   a.spins = s.d_spins;
   a.hot = s.d_hot;
   a.cold = s.d_cold;
+  a.tfound = s.d_tf;
   a.wlh = s.d_wlh;
   a.extra = s.d_extra;
   a.cap = s.cap;
@@ -627,6 +632,8 @@ int sadmc_init(sadmc_ctx *c) {
     HIPCHECK(c, hipMemsetAsync(s.d_hot, 0, sizeof(HotBin) * nb, c->stream));
     HIPCHECK(c, hipMalloc(&s.d_cold, sizeof(ColdBin) * nb));
     HIPCHECK(c, hipMemsetAsync(s.d_cold, 0, sizeof(ColdBin) * nb, c->stream));
+    HIPCHECK(c, hipMalloc(&s.d_tf, sizeof(uint64_t) * nb));
+    HIPCHECK(c, hipMemsetAsync(s.d_tf, 0, sizeof(uint64_t) * nb, c->stream));
     if (s.p.method == SADMC_WL || s.p.method == SADMC_INV_T_WL) {
       HIPCHECK(c, hipMalloc(&s.d_wlh, sizeof(uint64_t) * nb));
       HIPCHECK(c, hipMemsetAsync(s.d_wlh, 0, sizeof(uint64_t) * nb, c->stream));
@@ -1492,7 +1499,7 @@ int sadmc_upload_raw(sadmc_ctx *c, int32_t set, const sadmc_walker_state *states
     const size_t nb = (size_t)s.W * s.cap;
     std::vector<HotBin> h(nb);
     std::vector<ColdBin> cb(nb);
-    std::vector<uint64_t> wl(nb);
+    std::vector<uint64_t> tf(nb), wl(nb);
     for (size_t k = 0; k < nb; k++) {
       h[k].lnw = bins[k].lnw;
       h[k].hist = bins[k].histogram;
@@ -1500,12 +1507,12 @@ int sadmc_upload_raw(sadmc_ctx *c, int32_t set, const sadmc_walker_state *states
       cb[k].esq = bins[k].energy_squared_total;
       cb[k].rt = bins[k].round_trips;
       cb[k].vep = bins[k].visit_epoch;
-      cb[k].tfound = bins[k].t_found;
-      cb[k].pad = 0;
+      tf[k] = bins[k].t_found;
       wl[k] = bins[k].wl_hist;
     }
     HIPCHECK(c, hipMemcpy(s.d_hot, h.data(), sizeof(HotBin) * nb, hipMemcpyHostToDevice));
     HIPCHECK(c, hipMemcpy(s.d_cold, cb.data(), sizeof(ColdBin) * nb, hipMemcpyHostToDevice));
+    HIPCHECK(c, hipMemcpy(s.d_tf, tf.data(), sizeof(uint64_t) * nb, hipMemcpyHostToDevice));
     if (s.d_wlh) HIPCHECK(c, hipMemcpy(s.d_wlh, wl.data(), sizeof(uint64_t) * nb, hipMemcpyHostToDevice));
   }
   if (coords && s.p.system != SADMC_ISING) {

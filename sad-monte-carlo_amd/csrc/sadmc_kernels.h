@@ -166,7 +166,6 @@ __global__ __launch_bounds__(64) void k_init(SetArgs a, double e_lo) {
   Engine<SYS, KMAX, PREC, METH> e;
   e.load_system(a, walker, lane, lds + group * 3 * a.npad);
   e.from_params(walker, e_lo);
-  e.store(walker, true);
 }
 
 template <int SYS, int KMAX, int PREC, int METH>
