@@ -116,16 +116,20 @@ __global__ __launch_bounds__(512) void k_pt(SetArgs a, PtArgs p, uint64_t rounds
       e.s0 = m.rng0;
       e.s1 = m.rng1;
       for (int i = 0; i < p.steps; i++) {
-        double e2;
-        if (!e.cube_plan(p.d, p.sc, e2)) continue;
+        // selects instead of branches: the replicas of a wave would take
+        // the sides one after the other
+        double e2 = e.E;
+        const bool some = e.cube_plan(p.d, p.sc, e2);
         const double bde = (e2 - e.E) / m.T;
-        if (bde < 0.0 || gen_f64(e.s0, e.s1) < exp(-bde)) {
-          e.confirm();
-          m.acc += 1;
-        } else {
-          m.rej += 1;
-        }
-        pt_collect(m, e.E);
+        const bool acc = some & e.canonical_test(some, bde);
+        if (acc) e.confirm_system();
+        e.settle_energy(acc, e2, e.pdabse);
+        m.acc += acc ? 1 : 0;
+        m.rej += (some & !acc) ? 1 : 0;
+        const double te = m.te + e.E, tes = m.tes + e.E * e.E;
+        m.te = some ? te : m.te;
+        m.tes = some ? tes : m.tes;
+        m.ign += (some & (e.E >= 0.0)) ? 1 : 0;
       }
       if (lane == 0) {
         m.rng0 = e.s0;

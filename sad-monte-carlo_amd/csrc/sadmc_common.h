@@ -38,14 +38,28 @@ SADMC_HD void rng_seed(uint64_t seed, uint64_t &s0, uint64_t &s1) {
   s1 = splitmix_next(x);
 }
 
-// xoroshiro128+ next_u64, src/rng.rs:48-57.
+// xoroshiro128+ next_u64, src/rng.rs:48-57.  On the device in 32-bit halves:
+// the rotations are two funnel shifts each and the three-way xor one
+// instruction a half (11 instructions a draw instead of 15).
 SADMC_HD uint64_t rng_next(uint64_t &s0, uint64_t &s1) {
+#ifdef __HIP_DEVICE_COMPILE__
+  const uint64_t r = s0 + s1;
+  const uint32_t al = (uint32_t)s0, ah = (uint32_t)(s0 >> 32);
+  const uint32_t bl = (uint32_t)s1 ^ al, bh = (uint32_t)(s1 >> 32) ^ ah;
+  const uint32_t lo = __builtin_amdgcn_bitop3_b32(__builtin_amdgcn_alignbit(al, ah, 8), bl, bl << 16, 0x96);
+  const uint32_t hi = __builtin_amdgcn_bitop3_b32(__builtin_amdgcn_alignbit(ah, al, 8), bh,
+                                                  __builtin_amdgcn_alignbit(bh, bl, 16), 0x96);
+  s0 = ((uint64_t)hi << 32) | lo;
+  s1 = ((uint64_t)__builtin_amdgcn_alignbit(bl, bh, 27) << 32) | __builtin_amdgcn_alignbit(bh, bl, 27);
+  return r;
+#else
   uint64_t a = s0, b = s1;
   uint64_t r = a + b;
   b ^= a;
   s0 = rotl64(a, 24) ^ b ^ (b << 16);
   s1 = rotl64(b, 37);
   return r;
+#endif
 }
 
 // The 2^64-step jump of xoroshiro128+ (the published jump polynomial), as
@@ -91,7 +105,13 @@ SADMC_HD uint64_t uniform_index(uint64_t &s0, uint64_t &s1, uint64_t n) {
 // rng.gen::<f64>() (src/mc/energy.rs:465,489,498,508).
 SADMC_HD double gen_f64(uint64_t &s0, uint64_t &s1) {
   uint64_t v = rng_next(s0, s1);
+#ifdef __HIP_DEVICE_COMPILE__
+  // the same 53 bits, each half converted by itself; the sum is exact
+  const double lo = (double)((uint32_t)v & 0xFFFFF800u) * (1.0 / 18446744073709551616.0);
+  return __builtin_fma((double)(uint32_t)(v >> 32), 1.0 / 4294967296.0, lo);
+#else
   return (1.0 / 9007199254740992.0) * (double)(v >> 11);
+#endif
 }
 
 // Uniform::new(low, high) for f64, as rand 0.7's UniformFloat.
@@ -205,11 +225,18 @@ SADMC_HD double wca_pair_pressure(double r2, double rc2) {
 
 SADMC_HD double norm2(double x, double y, double z) { return x * x + y * y + z * z; }
 
-// Minimum-image component for two positions inside [0, L).
+// wca_pair with the fast reciprocal and a select, the same bits for every r2
+// (for those below 2^-766, where the reciprocals may differ, both terms are
+// NaN: s^6 and s^3 overflow).
+SADMC_DF double wca_pair_fast(double r2, double rc2) {
+  const double v = lj_pair_fast(r2) + 1.0;
+  return r2 < rc2 ? v : 0.0;
+}
+
+// Minimum-image component for two positions inside [0, L): d - L above
+// L/2, d + L below -L/2 (d - 0 is d).
 SADMC_HD double min_image(double d, double L, double halfL) {
-  if (d > halfL) return d - L;
-  if (d < -halfL) return d + L;
-  return d;
+  return d - (__builtin_fabs(d) > halfL ? __builtin_copysign(L, d) : 0.0);
 }
 
 // src/system/optcell.rs:277-309.
@@ -222,6 +249,15 @@ SADMC_HD double put_in_cell(double r, double L) {
     while (r >= L) r -= L;
   }
   return r;
+}
+
+// put_in_cell with its first step as selects; a second one is hardly ever
+// needed.
+SADMC_DF double put_in_cell_step(double r, double L) {
+  const bool neg = r < 0.0, big = r >= L;
+  const double a = neg ? r + L : big ? r - L : r;
+  if (__builtin_expect((neg & (a < 0.0)) | (big & (a >= L)), 0)) return put_in_cell(r, L);
+  return a;
 }
 
 }  // namespace sadmc

@@ -74,6 +74,7 @@ struct SetArgs {
   int32_t method, move_plan, has_min_e, has_max_e, has_min_gamma;
   int32_t refresh, collect_pressure, precision, move_kind;
   double method_param, move_param, min_e, max_e, rc2, width, inv_width;
+  double floor_e, ceil_e;  // min_e and max_e, or -inf and +inf without them
   const uint16_t *mlp;  // learned proposal: 1377 BF16 weights, or null
 };
 
@@ -143,6 +144,10 @@ struct Engine {
   // registers for the rest of the state.
   static constexpr bool kLdsPos = MV == 1 || SYS == SYS_WCA || KMAX >= 8;
   double x[KMAX], y[KMAX], z[KMAX];
+  // The slots a pair loop runs without asking for K, so that their chains
+  // interleave: K > KMAX/2 always, and up to 4 slots the one too many is
+  // cheaper than a branch.
+  static constexpr int kFirst = KMAX <= 4 ? KMAX : KMAX / 2 + 1;
   SADMC_DF double xk(int k) const { return kLdsPos ? lx[lane + G * k] : x[k]; }
   SADMC_DF double yk(int k) const { return kLdsPos ? ly[lane + G * k] : y[k]; }
   SADMC_DF double zk(int k) const { return kLdsPos ? lz[lane + G * k] : z[k]; }
@@ -164,9 +169,11 @@ struct Engine {
   double btop;  // bmin + width * len, the upper edge of the bins
   // SAD (tF and N_s are whole and exact); rtF, rNs = 1 / tF, 1 / N_s and
   // gzero (gamma is 0) follow lam, tF and N_s, which change rarely; tl_now:
-  // tL was set in this move.  min_T, tL, the largest t_found and WCA's
-  // has_pressure are touched so rarely that they stay in the walker's record.
-  double too_lo, too_hi, lam, tF, Ns, rtF, rNs, lnw_hi;
+  // tL was set in this move; tmax: the largest t_found in the range.  What a
+  // walker below too_lo needs each move is here too: one such walker, which
+  // can stay there for a whole launch, holds up its wave and so the launch.
+  // tL and WCA's has_pressure, only ever written, stay in the walker's record.
+  double too_lo, too_hi, lam, min_T, tF, Ns, rtF, rNs, lnw_lo, lnw_hi, tmax;
   bool gzero, tl_now;
   uint64_t highest;
   int32_t ilo, ihi;
@@ -183,6 +190,7 @@ struct Engine {
   uint64_t c_hist, c_wlh;
   double c_etot, c_esq;
   uint64_t c_rt, c_vep;
+  int32_t from_i;  // the bin this move started in
   // periodic triggers
   double next_check, next_press;  // in moves
   // pending move
@@ -192,15 +200,20 @@ struct Engine {
   const uint16_t *PW;
   float *XC;
   double lnh;
-  // this move's SAD gamma, computed while the proposed bin's record loads
-  // (again if the move changes lambda or N_s), and the next uniform with
-  // the generator state after drawing it, computed before it is needed
+  // this move's SAD gamma (computed again if the move changes lambda or N_s),
+  // and the next uniform with the generator state after drawing it, computed
+  // while the proposed bin's record loads
   double gpre, spec_u;
   uint64_t spec0, spec1;
-  // sqrt(1 / moves) for the group's next G moves: lane l holds the value of
-  // move rs_first + l; rs_next counts the moves served from it (G = empty)
-  double rs_lane;
-  int32_t rs_next;
+  // SAD's gamma for the group's next G moves, one per lane; g_next counts the
+  // moves served from it (G: none left)
+  double g_lane;
+  int32_t g_next;
+  // sqrt(1 / moves) for the wave's next 64 moves, one per lane, while its
+  // walkers all stand at one move number (rs_same; as they do unless they
+  // were uploaded at different ones)
+  double rs_wave;
+  bool rs_same;
 
   // ---------------------------------------------------------------- setup
   SADMC_DF void load_system(const SetArgs &a, int walker, int lane_in_group, double *lds_group) {
@@ -223,6 +236,11 @@ struct Engine {
       const double *P = a.pos + (int64_t)walker * 3 * a.npad;
 #pragma unroll
       for (int k = 0; k < KMAX; k++) {
+        if (!kLdsPos) {
+          x[k] = 0.0;
+          y[k] = 0.0;
+          z[k] = 0.0;
+        }
         if (k < K) {
           int j = lane + G * k;
           const double vx = P[j], vy = P[a.npad + j], vz = P[2 * a.npad + j];
@@ -248,7 +266,6 @@ struct Engine {
     E = w.E;
     err = w.error;
     tm = (double)w.moves;
-    rs_next = 1 << 30;
     accepted = w.accepted_moves;
     acc_rate = w.acceptance_rate;
     tscale = w.translation_scale;
@@ -265,6 +282,8 @@ struct Engine {
       too_lo = w.too_lo;
       too_hi = w.too_hi;
       lam = w.latest_parameter;
+      min_T = w.min_T;
+      tmax = (double)w.tmax;
       tF = (double)w.tF;
       Ns = (double)w.num_states;
       highest = w.highest_hist;
@@ -286,6 +305,7 @@ struct Engine {
     }
     usc = SYS == SYS_ISING ? 0.0 : uniform_scale(-tscale, tscale);
     btop = bmin + args().width * (double)len;
+    g_next = G;
     if (METH == M_SAD) gamma_changed();
     cur_p = -1;
     if (!status) {
@@ -307,6 +327,7 @@ struct Engine {
         w.tF = (uint64_t)tF;
         w.num_states = (uint64_t)Ns;
         w.highest_hist = highest;
+        w.tmax = (uint64_t)tmax;
       }
       if (METH == M_SAMC || METH == M_WL) w.t0 = t0;
       if (METH == M_WL) {
@@ -391,7 +412,7 @@ struct Engine {
   // The current bin's record goes back to memory when the walker leaves the
   // bin or the launch ends (every read in between takes the registers).
   SADMC_DF void write_back() {
-    if (cur_p >= 0) {
+    if (lane == 0 && cur_p >= 0) {
       HotBin hb;
       hb.lnw = c_lnw;
       hb.hist = c_hist;
@@ -425,7 +446,9 @@ struct Engine {
   // window change) and reload the values cached at those indices.  An index
   // past the bins is left for move_once to report where the reference would
   // index out of bounds.
-  SADMC_DF void refresh_indices() {
+  // plo, phi: the physical bins whose ln w lnw_lo and lnw_hi already hold (a
+  // window that grew at the front moves the indices, not the records).
+  SADMC_DF void refresh_indices(int32_t plo = -1, int32_t phi = -1) {
     int32_t i = e_index(E);
     cur_i = i;
     if (i < len) {
@@ -438,7 +461,8 @@ struct Engine {
     if (METH == M_SAD) {
       ilo = e_index(too_lo);
       ihi = e_index(too_hi);
-      lnw_hi = ihi < len ? lnw_at(base + ihi) : 0.0;
+      if (ilo >= len || base + ilo != plo) lnw_lo = ilo < len ? lnw_at(base + ilo) : 0.0;
+      if (ihi >= len || base + ihi != phi) lnw_hi = ihi < len ? lnw_at(base + ihi) : 0.0;
     }
   }
 
@@ -466,6 +490,8 @@ struct Engine {
   // A window without room stops the walker.
   SADMC_DF void prepare_for_range(double lo, double hi) {
     bool front = false, grew = false;
+    const int32_t plo = METH == M_SAD && ilo < len ? base + ilo : -1;
+    const int32_t phi = METH == M_SAD && ihi < len ? base + ihi : -1;
     while (status == 0 && lo < bmin) {
       if (base == 0) {
         status = SADMC_WS_CAPACITY;
@@ -490,7 +516,7 @@ struct Engine {
       }
     }
     btop = bmin + args().width * (double)len;
-    if (status == 0 && (front || (grew && !indices_valid()))) refresh_indices();
+    if (status == 0 && (front || (grew && !indices_valid()))) refresh_indices(plo, phi);
     if (status == 0 && (front || grew) && SYS != SYS_ISING && args().refresh <= 0) {
       uint64_t P = (uint64_t)len * (uint64_t)len * 1000ULL;
       next_check = (double)((moves() / P + 1) * P);
@@ -525,13 +551,104 @@ struct Engine {
         if (SYS == SYS_LJ) {
           acc += lj_pair(norm2(xi - lx[j], yi - ly[j], zi - lz[j]));
         } else {
-          acc += wca_pair(norm2(min_image(xi - lx[j], L, halfL), min_image(yi - ly[j], L, halfL),
-                                min_image(zi - lz[j], L, halfL)),
-                          args().rc2);
+          acc += wca_pair_fast(norm2(min_image(xi - lx[j], L, halfL), min_image(yi - ly[j], L, halfL),
+                                     min_image(zi - lz[j], L, halfL)),
+                               args().rc2);
         }
       }
     }
     return group_sum(acc, G);
+  }
+
+  // The full energy of the group that lane `leader` belongs to, by the whole
+  // wave (all 64 lanes running, the tiles of the wave's groups side by side in
+  // LDS): lane v of group c takes the pairs (i, j) with i = v, v + G, ... and
+  // j = c, c + 64/G, ..., and each lane then adds the terms of its v in the
+  // order of j, which is the order of full_energy, so the bits are the same.
+  // A term left out (j >= i) adds +0, which changes no sum here (none is
+  // -0: they start at +0).
+  //
+  // The walkers of a wave need a new energy one by one, when their own error
+  // estimate trips (LJ every 10 N accepted moves, WCA every 10), and a group
+  // alone runs through the N^2/2 pairs with 64 - G lanes idle.
+  SADMC_DF double wave_full_energy(int leader) const {
+    const int R = 64 / G, c = (int)(threadIdx.x & 63) / G;
+    const double *X = lx + (leader / G - c) * 3 * args().npad, *Y = X + args().npad, *Z = Y + args().npad;
+    const double Lw = SYS == SYS_WCA ? __shfl(L, leader, 64) : 0.0, hw = 0.5 * Lw;
+    constexpr int U = 4;  // terms in flight per lane
+    double acc = 0.0;
+#pragma unroll 1
+    for (int i0 = 0; i0 < n; i0 += G) {
+      const int i = i0 + lane;
+      const int jend = i < n ? i : 0;  // this lane's pairs: j < jend
+      const int jmax = i0 + G - 1 < n - 1 ? i0 + G - 1 : n - 1;
+      const double xi = X[jend], yi = Y[jend], zi = Z[jend];
+#pragma unroll 1
+      for (int j0 = 0; j0 < jmax; j0 += R * U) {
+        double t[U];
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+          const int j = j0 + u * R + c;
+          const bool ok = j < jend;
+          const int jj = ok ? j : 0;
+          double v;
+          if (SYS == SYS_LJ) {
+            v = lj_pair_fast(norm2(xi - X[jj], yi - Y[jj], zi - Z[jj]));
+          } else {
+            v = wca_pair_fast(norm2(min_image(xi - X[jj], Lw, hw), min_image(yi - Y[jj], Lw, hw),
+                                    min_image(zi - Z[jj], Lw, hw)),
+                              args().rc2);
+          }
+          t[u] = ok ? v : 0.0;
+        }
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+          if (j0 + u * R < jmax) {
+            if (GC > 0) {
+#pragma unroll
+              for (int q = 0; q < R; q++) acc += __shfl(t[u], q * G + lane, 64);
+            } else {
+              for (int q = 0; q < R; q++) acc += __shfl(t[u], q * G + lane, 64);
+            }
+          }
+        }
+      }
+    }
+    return group_sum(acc, G);
+  }
+
+  // A group of lanes without a walker (the last wave's, or a wave that holds
+  // fewer than it could): it runs no moves and helps in wave_full_energy.
+  SADMC_DF void load_idle(const SetArgs &a, int lane_in_group, double *lds_group) {
+    Ap = &a;
+    lane = lane_in_group;
+    G = GC ? GC : a.G;
+    K = a.K;
+    n = a.n;
+    lx = lds_group;
+    status = SADMC_WS_OK + 100;
+    L = 0.0;
+  }
+
+  // Full energies for the walkers with `need`, each the value of
+  // full_energy (NaN sums, where the fast reciprocal may differ, included).
+  SADMC_DF void full_energies(bool need) {
+    uint64_t todo = __ballot(need);
+    if (!todo) return;
+    bool serial = need;
+    if (SYS != SYS_ISING && G < 64 && __ballot(1) == ~0ULL) {
+      const int mine = (int)(threadIdx.x & 63) / G;
+      while (todo) {
+        const int leader = (int)__builtin_ctzll(todo);
+        todo &= ~(((1ULL << G) - 1) << (leader / G * G));
+        const double e = wave_full_energy(leader);
+        if (leader / G == mine) {
+          E = e;
+          serial = SYS == SYS_LJ && e != e;
+        }
+      }
+    }
+    if (__builtin_expect(serial, 0)) E = full_energy();
   }
 
   // wca.rs:202-218 virial, ordered pairs, lane-group order.
@@ -555,8 +672,22 @@ struct Engine {
   // ising.rs:104-119.
   SADMC_DF bool ising_plan(double &e2) {
     const int N = n;
-    int i = (int)sample_zone(s0, s1, (uint32_t)N, args().zone_site);
-    int j = (int)sample_zone(s0, s1, (uint32_t)N, args().zone_site);
+    // sample_zone twice, in one loop: the zone is conservative (it refuses
+    // half of the draws at N = 8), and every walker of the wave waits for the
+    // one with the most refusals, of both draws together here instead of of
+    // each
+    int i = 0, j = -1;
+    bool first = true;
+    do {
+      const uint64_t v = rng_next(s0, s1);
+      const uint64_t a = (uint64_t)(uint32_t)v * (uint32_t)N;
+      const uint64_t b = (uint64_t)(uint32_t)(v >> 32) * (uint32_t)N + (a >> 32);
+      const bool ok = ((b << 32) | (uint32_t)a) <= args().zone_site;
+      const int site = (int)(b >> 32);
+      j = (ok & !first) ? site : j;
+      i = (ok & first) ? site : i;
+      first = first & !ok;
+    } while (j < 0);
     int jp = j + 1 == N ? 0 : j + 1;
     int jm = j == 0 ? N - 1 : j - 1;
     int ip = i + 1 == N ? 0 : i + 1;
@@ -574,10 +705,11 @@ struct Engine {
   // energy difference.
   SADMC_DF bool particle_plan(double d, double sc, double &e2) {
     int w = (int)sample_zone(s0, s1, (uint32_t)n, args().zone_n);
+    const double fx = lx[w], fy = ly[w], fz = lz[w];
+    __builtin_amdgcn_sched_barrier(0);  // the LDS reads run under the draws
     double ux = uniform_sample(s0, s1, -d, sc);
     double uy = uniform_sample(s0, s1, -d, sc);
     double uz = uniform_sample(s0, s1, -d, sc);
-    double fx = lx[w], fy = ly[w], fz = lz[w];
     double tx, ty, tz;
     // a move past the wall still runs through the sums below: its wave does
     // so anyway while any of its walkers moves inside
@@ -589,29 +721,34 @@ struct Engine {
       double r2to = norm2(tx, ty, tz), r2from = norm2(fx, fy, fz);
       some = !(r2to > R2 && r2to > r2from);
     } else {
-      tx = put_in_cell(fx + ux, L);
-      ty = put_in_cell(fy + uy, L);
-      tz = put_in_cell(fz + uz, L);
+      tx = put_in_cell_step(fx + ux, L);
+      ty = put_in_cell_step(fy + uy, L);
+      tz = put_in_cell_step(fz + uz, L);
     }
     double acc = 0.0, accabs = 0.0;
     if (SYS == SYS_LJ) {
       acc = lj_lane_diff(w, tx, ty, tz, fx, fy, fz);
     } else {
+      auto slot = [&](int k) {
+        const int j = lane + G * k;
+        const bool use = (j < n) & (j != w);
+        const int jr = 2 * k > KMAX && j >= n ? 0 : j;  // as in lj_lane_sum
+        const double xj = lx[jr], yj = ly[jr], zj = lz[jr];
+        const double vn = wca_pair_fast(norm2(min_image(xj - tx, L, halfL), min_image(yj - ty, L, halfL),
+                                              min_image(zj - tz, L, halfL)),
+                                        args().rc2);
+        const double vo = wca_pair_fast(norm2(min_image(xj - fx, L, halfL), min_image(yj - fy, L, halfL),
+                                              min_image(zj - fz, L, halfL)),
+                                        args().rc2);
+        const double na = acc + (vn - vo), nb = accabs + (vn + vo);
+        acc = use ? na : acc;
+        accabs = use ? nb : accabs;
+      };
 #pragma unroll
-      for (int k = 0; k < KMAX; k++) {
-        if (k < K) {
-          const int j = lane + G * k;
-          const bool use = j < n && j != w;
-          double vn = wca_pair(norm2(min_image(xk(k) - tx, L, halfL), min_image(yk(k) - ty, L, halfL),
-                                     min_image(zk(k) - tz, L, halfL)),
-                               args().rc2);
-          double vo = wca_pair(norm2(min_image(xk(k) - fx, L, halfL), min_image(yk(k) - fy, L, halfL),
-                                     min_image(zk(k) - fz, L, halfL)),
-                               args().rc2);
-          const double na = acc + (vn - vo), nb = accabs + (vn + vo);
-          acc = use ? na : acc;
-          accabs = use ? nb : accabs;
-        }
+      for (int k = 0; k < kFirst; k++) slot(k);
+      if (kFirst < KMAX && K > kFirst) {
+#pragma unroll
+        for (int k = kFirst; k < KMAX; k++) slot(k);
       }
     }
     double e = E + group_sum(acc, G);
@@ -651,24 +788,29 @@ struct Engine {
   // divergent branch per atom.
   SADMC_DF double lj_lane_sum(int w, double tx, double ty, double tz, double fx, double fy, double fz) {
     double acc = 0.0;
-#pragma unroll
-    for (int k = 0; k < KMAX; k++) {
-      if (k < K) {
-        const int j = lane + G * k;
-        const bool use = j < n && j != w;
-        double t;
-        if (PREC == 1) {
-          const float an = (float)(xk(k) - tx), bn = (float)(yk(k) - ty), cn = (float)(zk(k) - tz);
-          const float ao = (float)(xk(k) - fx), bo = (float)(yk(k) - fy), co = (float)(zk(k) - fz);
-          t = (double)lj_pair_f32_fast(an * an + bn * bn + cn * cn) -
-              (double)lj_pair_f32_fast(ao * ao + bo * bo + co * co);
-        } else {
-          t = lj_pair_fast(norm2(xk(k) - tx, yk(k) - ty, zk(k) - tz)) -
-              lj_pair_fast(norm2(xk(k) - fx, yk(k) - fy, zk(k) - fz));
-        }
-        const double na = acc + t;
-        acc = use ? na : acc;
+    auto slot = [&](int k) {
+      const int j = lane + G * k;
+      const bool use = (j < n) & (j != w);
+      // slots that K may not reach read atom 0 (and are dropped)
+      const int jr = 2 * k > KMAX && j >= n ? 0 : j;
+      const double xj = kLdsPos ? lx[jr] : x[k], yj = kLdsPos ? ly[jr] : y[k], zj = kLdsPos ? lz[jr] : z[k];
+      double t;
+      if (PREC == 1) {
+        const float an = (float)(xj - tx), bn = (float)(yj - ty), cn = (float)(zj - tz);
+        const float ao = (float)(xj - fx), bo = (float)(yj - fy), co = (float)(zj - fz);
+        t = (double)lj_pair_f32_fast(an * an + bn * bn + cn * cn) -
+            (double)lj_pair_f32_fast(ao * ao + bo * bo + co * co);
+      } else {
+        t = lj_pair_fast(norm2(xj - tx, yj - ty, zj - tz)) - lj_pair_fast(norm2(xj - fx, yj - fy, zj - fz));
       }
+      const double na = acc + t;
+      acc = use ? na : acc;
+    };
+#pragma unroll
+    for (int k = 0; k < kFirst; k++) slot(k);
+    if (kFirst < KMAX && K > kFirst) {
+#pragma unroll
+      for (int k = kFirst; k < KMAX; k++) slot(k);
     }
     return acc;
   }
@@ -745,7 +887,7 @@ struct Engine {
   SADMC_DF bool sad_lnw(double e, double &out) {
     if (ilo < 0 || ilo >= len || ihi < 0 || ihi >= len) return false;
     if (e < too_lo) {
-      out = lnw_at(base + ilo) + (e - too_lo) / rec().min_T;
+      out = lnw_lo + (e - too_lo) / min_T;
       return true;
     }
     if (e > too_hi) {
@@ -811,37 +953,48 @@ struct Engine {
     return particle_plan(d, sc, e2);
   }
 
-  // lj.rs:106-123.
-  SADMC_DF void lj_set_energy(double new_e) {
-    double nn = (double)n;
-    double new_error = fabs(new_e) > fabs(E) ? fabs(new_e) * 1e-15 * nn : fabs(E) * 1e-15 * nn;
-    err = new_error + err;
-    if (err > fabs(new_e) * 1e-14 * nn * nn) {
-      err *= 0.0;
-      E = full_energy();
+  // lj.rs:106-123 and wca.rs:164-180 for a walker with `acc`: the new energy
+  // is taken over unless the running error estimate has grown past its bound,
+  // which asks for a full recomputation (true).
+  SADMC_DF bool take_energy(bool acc, double new_e, double dabse) {
+    if (SYS == SYS_ISING || args().refresh > 0) {
+      E = acc ? new_e : E;
+      return false;
+    }
+    const double nn = (double)n, ae = fabs(new_e);
+    double ne;
+    bool trip;
+    if (SYS == SYS_LJ) {
+      ne = (ae > fabs(E) ? ae * 1e-15 * nn : fabs(E) * 1e-15 * nn) + err;
+      trip = ne > ae * 1e-14 * nn * nn;
+      ne = trip ? ne * 0.0 : ne;
     } else {
-      E = new_e;
+      const double single = dabse > ae ? 1e-14 * dabse * nn : 1e-14 * ae * nn;
+      ne = err + single * nn;
+      trip = ne > ae * 1e-13 * nn * nn;
+    }
+    err = acc ? ne : err;
+    E = acc && !trip ? new_e : E;
+    return acc && trip;
+  }
+  // After the recomputation (wca.rs:175-177).
+  SADMC_DF void took_full_energy() {
+    if (SYS == SYS_WCA) err = 1e-15 * E * (double)n;
+  }
+  // take_energy with the recomputations shared by the wave.
+  SADMC_DF void settle_energy(bool acc, double new_e, double dabse) {
+    const bool trip = take_energy(acc, new_e, dabse);
+    if (__builtin_expect(__any(trip), 0)) {
+      full_energies(trip);
+      if (trip) took_full_energy();
     }
   }
 
-  // wca.rs:164-180.
-  SADMC_DF void wca_set_energy(double new_e, double dabse) {
-    double nn = (double)n;
-    double single = dabse > fabs(new_e) ? 1e-14 * dabse * nn : 1e-14 * fabs(new_e) * nn;
-    err += single * nn;
-    if (err > fabs(new_e) * 1e-13 * nn * nn) {
-      E = full_energy();
-      err = 1e-15 * E * nn;
-    } else {
-      E = new_e;
-    }
-  }
-
-  // ConfirmSystem::confirm: ising.rs:94-101, lj.rs:338-358, wca.rs:276-301.
-  SADMC_DF void confirm() {
+  // The part of ConfirmSystem::confirm (ising.rs:94-101, lj.rs:338-358,
+  // wca.rs:276-301) that moves the atom.
+  SADMC_DF void confirm_system() {
     if (SYS == SYS_ISING) {
       spins ^= (1ULL << pw);
-      E = pe;
       return;
     }
     int owner = pw & (G - 1);
@@ -860,12 +1013,13 @@ struct Engine {
       lz[pw] = ptz;
     }
     __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-    if (args().refresh > 0) {
-      E = pe;
-    } else if (SYS == SYS_LJ) {
-      lj_set_energy(pe);
-    } else {
-      wca_set_energy(pe, pdabse);
+  }
+  // The whole of it, for callers whose groups confirm on their own.
+  SADMC_DF void confirm() {
+    confirm_system();
+    if (take_energy(true, pe, pdabse)) {
+      E = full_energy();
+      took_full_energy();
     }
   }
 
@@ -890,17 +1044,20 @@ struct Engine {
     q = __builtin_fma(__builtin_fma(-b, q, a), y, q);
     return __builtin_fma(__builtin_fma(-b, q, a), y, q);
   }
-  SADMC_DF double sad_gamma() const {
-    const double q = quot(tm, tF, rtF);
-    const double g = (lam + q) / (lam + quot(tm, Ns, rNs) * q);
+  SADMC_DF double sad_gamma(double t) const {
+    const double q = quot(t, tF, rtF);
+    const double g = (lam + q) / (lam + quot(t, Ns, rNs) * q);
     return gzero ? 0.0 : g;
   }
-  // After a change of lam, tF or Ns.
+  // After a change of lam, tF or Ns (during move tm): the reciprocals, and
+  // the gammas of the moves from tm on that the lanes hold.
   SADMC_DF void gamma_changed() {
     rtF = 1.0 / tF;
     rNs = 1.0 / Ns;
     gzero = lam * tF * Ns == 0.0;
+    g_lane = sad_gamma(tm + (double)(lane - (g_next - 1)));
   }
+  SADMC_DF double gamma_now() const { return G == 1 ? g_lane : __shfl(g_lane, g_next - 1, G); }
 
   // Draw the next uniform ahead of the test that may use it.
   SADMC_DF void spec_draw() {
@@ -926,66 +1083,63 @@ struct Engine {
     const double est = (double)__builtin_amdgcn_exp2f((float)t);
     const double band = est * (1e-5 - 1e-6 * t);
     bool rejected = spec_u > est + band;
-    if (__builtin_expect(need && !rejected && !(spec_u < est - band), 0)) rejected = spec_u > exp(x);
-    return need && rejected;
+    if (__builtin_expect(need & !rejected & !(spec_u < est - band), 0)) rejected = spec_u > exp(x);
+    return need & rejected;
+  }
+  // tempering.rs:101-104: `bde < 0 || u < exp(-bde)`, the uniform drawn only
+  // for bde not below 0 (and `some`); settled as in mh_test.
+  SADMC_DF bool canonical_test(bool some, double bde) {
+    const bool need = some & !(bde < 0.0);
+    spec_draw();
+    s0 = need ? spec0 : s0;
+    s1 = need ? spec1 : s1;
+    double t = bde * -1.4426950408889634;
+    t = t < -1000.0 ? -1000.0 : t;
+    const double est = (double)__builtin_amdgcn_exp2f((float)t);
+    const double band = est * (1e-5 - 1e-6 * t);
+    bool take = spec_u < est - band;
+    if (__builtin_expect(need & !take & !(spec_u > est + band), 0)) take = spec_u < exp(-bde);
+    return !need | take;
   }
   // Metropolis-Hastings test on the log acceptance ratio.
-  SADMC_DF bool reject_lr(bool go, double lr) { return mh_test(go && lr < 0.0, lr); }
+  SADMC_DF bool reject_lr(bool go, double lr) { return mh_test(go & (lr < 0.0), lr); }
   // ln w(e) with the SAD clamped extension (energy.rs:445-463); `inside` is
   // the bin's ln w.
   SADMC_DF double sad_lnw_ext(double e, double inside) const {
     double v = e > too_hi ? lnw_hi : inside;
-    if (__builtin_expect(e < too_lo, 0)) v = lnw_at(base + ilo) + (e - too_lo) / rec().min_T;
+    if (__builtin_expect(e < too_lo, 0)) v = lnw_lo + (e - too_lo) / min_T;
     return v;
   }
 
-  // energy.rs:440-512.  `r2` is the record of the proposed bin; nothing
-  // happens for a walker without a move to test (`go` false).  The
-  // learned move adds ln H to the exponent (the tests are the reference's
-  // when ln H = 0).
-  SADMC_DF bool reject_move(bool go, double e1, double e2, double r2_lnw, uint64_t r2_hist) {
-    if (MV == 1) {
-      if (METH == M_SAD) {
-        const double lnw1 = sad_lnw_ext(e1, c_lnw), lnw2 = sad_lnw_ext(e2, r2_lnw);
-        bool rejected = reject_lr(go, lnw1 - lnw2 + lnh);
-        if (__builtin_expect(go && !rejected && r2_hist == 0, 0) && e2 < too_hi && e2 > too_lo) {
-          lam = (too_hi - too_lo) / rec().min_T;
-          Ns += 1.0;
-          set_tL();
-          gamma_changed();
-          gpre = sad_gamma();
-        }
-        return rejected;
-      } else if (METH == M_SAMC) {
-        return reject_lr(go, c_lnw - r2_lnw + lnh);
-      } else if (METH == M_WL) {
-        bool rejected = reject_lr(go, c_lnw - r2_lnw + lnh);
-        if (go && method != SADMC_SAMC && !rejected && r2_hist == 0 && wl_lowest > 0) wl_Ns += 1.0;
-        return rejected;
-      } else {
-        return reject_lr(go, (e1 - e2) / args().method_param + lnh);
-      }
+  // energy.rs:440-512 on l1 and l2, ln w at the two energies (with SAD's
+  // extension outside its range), and the proposed bin's count; nothing
+  // happens for a walker without a move to test (`go` false).  The learned
+  // move adds ln H to the exponent (the tests are the reference's when
+  // ln H = 0).
+  SADMC_DF bool reject_move(bool go, double e1, double e2, double l1, double l2, uint64_t r2_hist) {
+    bool rejected;
+    if (METH == M_CAN) {
+      if (MV == 1) return reject_lr(go, (e1 - e2) / args().method_param + lnh);
+      return mh_test(go & (e1 < e2), (e1 - e2) / args().method_param);
     }
+    if (MV == 1) {
+      rejected = reject_lr(go, l1 - l2 + lnh);
+    } else {
+      rejected = mh_test(go & (l2 > l1), l1 - l2);
+    }
+    const bool found = go & !rejected & (r2_hist == 0);
     if (METH == M_SAD) {
-      const double lnw1 = sad_lnw_ext(e1, c_lnw), lnw2 = sad_lnw_ext(e2, r2_lnw);
-      bool rejected = mh_test(go && lnw2 > lnw1, lnw1 - lnw2);
-      if (__builtin_expect(go && !rejected && r2_hist == 0, 0) && e2 < too_hi && e2 > too_lo) {
-        lam = (too_hi - too_lo) / rec().min_T;
+      if (__builtin_expect(found, 0) && e2 < too_hi && e2 > too_lo) {
+        lam = (too_hi - too_lo) / min_T;
         Ns += 1.0;
         set_tL();
         gamma_changed();
-        gpre = sad_gamma();
+        gpre = gamma_now();
       }
-      return rejected;
-    } else if (METH == M_SAMC) {
-      return mh_test(go && r2_lnw > c_lnw, c_lnw - r2_lnw);
     } else if (METH == M_WL) {
-      bool rejected = mh_test(go && r2_lnw > c_lnw, c_lnw - r2_lnw);
-      if (go && method != SADMC_SAMC && !rejected && r2_hist == 0 && wl_lowest > 0) wl_Ns += 1.0;
-      return rejected;
-    } else {
-      return mh_test(go && e1 < e2, (e1 - e2) / args().method_param);
+      if (found && method != SADMC_SAMC && wl_lowest > 0) wl_Ns += 1.0;
     }
+    return rejected;
   }
 
   // Running max of t_found over logical bins [a, b].
@@ -1016,27 +1170,26 @@ struct Engine {
       m = t > m ? t : m;
     }
     m = group_max_u64(m);
-    if (m > rec().tmax) rec().tmax = m;
+    tmax = (double)m > tmax ? (double)m : tmax;
   }
 
   // energy.rs:514-636 for the current bin (logical i = cur_i).
   SADMC_DF void update_sad(double E_, int32_t i) {
     const double E = E_;
-    if (!(too_lo > too_hi || E < too_lo || E > too_hi)) {
-      c_lnw += gpre;
-      if (cur_p == base + ihi) lnw_hi = c_lnw;
-    }
-    if (__builtin_expect(c_hist > highest || tl_now, 0)) update_sad_range(E, i);
+    const bool in = !((too_lo > too_hi) | (E < too_lo) | (E > too_hi));
+    c_lnw = in ? c_lnw + gpre : c_lnw;
+    lnw_lo = (in & (i == ilo)) ? c_lnw : lnw_lo;
+    lnw_hi = (in & (i == ihi)) ? c_lnw : lnw_hi;
+    if (__builtin_expect((c_hist > highest) | tl_now, 0)) update_sad_range(E, i);
   }
   // The part of update_sad that a new highest count or a new tL needs.
   SADMC_DF void update_sad_range(double E, int32_t i) {
     if (c_hist > highest) {
       highest = c_hist;
-      // the cached ln w at too_hi and N_s change here only when the range
-      // grows; otherwise ln w at that bin changes only through the current
-      // bin, which the increment above already tracks
+      // the cached ln w at too_lo / too_hi and N_s change here only when
+      // the range grows; otherwise ln w at those bins changes only through
+      // the current bin, which the increment above already tracks
       bool grew = false;
-      const double min_T = rec().min_T;
       if ((E > too_hi && ihi >= len) || (E < too_lo && ilo >= len)) {
         status = SADMC_WS_INDEX;
       } else if (E > too_hi) {
@@ -1076,7 +1229,7 @@ struct Engine {
         // every bin below too_lo extends from the old ln w(too_lo): the bin
         // of too_lo itself comes last in energy order
         int32_t jlo = i > 0 ? i - 1 : 0, jhi = ilo + 1 < len ? ilo + 1 : len - 1;
-        const double vlo = lnw_at(base + ilo);
+        const double vlo = lnw_lo;
         uint32_t cnt = 0;
         for (int32_t j = jlo + lane; j <= jhi; j += G) {
           const double ej = i_energy(j);
@@ -1115,12 +1268,15 @@ struct Engine {
         too_lo = nl;
         ilo = ilo2;
       }
-      if (grew && status == 0) lnw_hi = lnw_at(base + ihi);
+      if (grew && status == 0) {
+        lnw_lo = lnw_at(base + ilo);
+        lnw_hi = lnw_at(base + ihi);
+      }
     }
     if (tl_now && status == 0 && (ilo >= len || ihi >= len)) status = SADMC_WS_INDEX;
     if (tl_now && status == 0) {
       const double old_tF = tF;
-      tF = (double)rec().tmax;
+      tF = tmax;
       if (old_tF != tF && args().move_plan == SADMC_ACCEPTANCE_RATE) {
         double s = acc_rate / args().move_param;
         s = s < 0.8 ? 0.8 : (s > 1.2 ? 1.2 : s);
@@ -1128,7 +1284,7 @@ struct Engine {
         if (SYS != SYS_ISING) usc = uniform_scale(-tscale, tscale);
       }
     }
-    gamma_changed();
+    if (tl_now) gamma_changed();
   }
 
   // energy.rs:638-756 (WL and 1/t-WL); SAMC after the 1/t switch.
@@ -1219,7 +1375,11 @@ struct Engine {
   // what does not need them is computed meanwhile.  What is common is written
   // as selects rather than branches, which the walkers of a wave would
   // otherwise take one after the other; the rare parts stay branches.
-  SADMC_DF void move_once() {
+  //
+  // A move is a proposal and a visit; in between the wave recomputes the
+  // energies that the proposals asked for (true) together.
+  // `step`: this move's lane in rs_wave (the same in the whole wave).
+  SADMC_DF bool propose(int step) {
     bool regrow = false;
     tm += 1.0;
     if (METH == M_SAD) tl_now = false;
@@ -1245,24 +1405,29 @@ struct Engine {
     }
     const double e1 = E;
     int32_t i1 = cur_i;
-    double rs;
-    if (SYS == SYS_ISING) {
-      rs = sqrt(1.0 / tm);
-    } else {
-      // each lane of the group computes one of the next G values at once
-      if (rs_next >= G) {
-        rs_lane = sqrt(1.0 / (tm + (double)lane));
-        rs_next = 0;
+    if (METH == M_SAD) {
+      if (g_next >= G) {
+        g_lane = sad_gamma(tm + (double)lane);
+        g_next = 0;
       }
-      rs = __shfl(rs_lane, rs_next, G);
-      rs_next += 1;
+      g_next += 1;
+      gpre = gamma_now();
     }
-    acc_rate *= 1.0 - rs;
+    double rs;
+    if (__builtin_expect(rs_same, 1)) {
+      const uint64_t b = __builtin_bit_cast(uint64_t, rs_wave);
+      const uint32_t lo = __builtin_amdgcn_readlane((int)(uint32_t)b, step);
+      const uint32_t hi = __builtin_amdgcn_readlane((int)(uint32_t)(b >> 32), step);
+      rs = __builtin_bit_cast(double, ((uint64_t)hi << 32) | lo);
+    } else {
+      rs = sqrt(1.0 / tm);
+    }
     double e2 = e1;
     bool go = plan_move(tscale, usc, e2);
-    if (args().has_max_e) go = go && !(e2 > args().max_e && e2 > e1);
-    if (args().has_min_e) go = go && !(e2 < args().min_e && e2 < e1);
-    if (__builtin_expect(regrow || (go && (e2 < bmin || e2 >= btop)), 0)) {
+    acc_rate *= 1.0 - rs;
+    // (bitwise on purpose, here and below: && and || become branches)
+    go = go & !((e2 > args().ceil_e) & (e2 > e1)) & !((e2 < args().floor_e) & (e2 < e1));
+    if (__builtin_expect(regrow | (go & ((e2 < bmin) | (e2 >= btop))), 0)) {
       double lo = go ? e2 : E, hi = lo;
       if (regrow) {
         lo = E < lo ? E : lo;
@@ -1271,49 +1436,64 @@ struct Engine {
       prepare_for_range(lo, hi);
     }
     i1 = go ? cur_i : i1;
-    const int32_t i2 = go ? e_index(e2) : cur_i;
-    if (status == 0 && (cur_p < 0 || (go && (!indices_valid() || (uint32_t)i2 >= (uint32_t)len))))
-      status = SADMC_WS_INDEX;
-    if (__builtin_expect(status == 0, 1)) finish_move(go, e1, e2, i1, i2, rs);
+    const int32_t i2 = e_index(go ? e2 : e1);
+    bool bad = (uint32_t)i2 >= (uint32_t)len;
+    if (METH == M_SAD) bad = bad | (ilo >= len) | (ihi >= len);
+    if (__builtin_expect((status == 0) & ((cur_p < 0) | (go & bad)), 0)) status = SADMC_WS_INDEX;
+    from_i = i1;
+    bool trip = false;
+    if (__builtin_expect(status == 0, 1)) trip = decide(go, e1, e2, i2, rs);
+    return trip;
   }
-
-  // The second half of a move: the test, the accepted move's bookkeeping and
-  // the update of the bin the walker is in.
-  SADMC_DF void finish_move(bool go, double e1, double e2, int32_t i1, int32_t i2, double rs) {
+  // The test and the accepted move.
+  SADMC_DF bool decide(bool go, double e1, double e2, int32_t i2, double rs) {
     const int32_t p2 = go ? base + i2 : cur_p;
     const HotBin hb = H[p2];
     const ColdBin cb = Cb[p2];
     uint64_t wl2 = 0;
     if (METH == M_WL) wl2 = WH[p2];
     // independent of the record being loaded
-    if (METH == M_SAD) gpre = sad_gamma();
     spec_draw();
+    double l1 = c_lnw, out2 = 0.0;
+    bool ext2 = false;
+    if (METH == M_SAD) {
+      l1 = sad_lnw_ext(e1, c_lnw);
+      out2 = sad_lnw_ext(e2, 0.0);
+      ext2 = (e2 < too_lo) | (e2 > too_hi);
+    }
     const bool same = p2 == cur_p;
-    const double w2 = same ? c_lnw : hb.lnw;
+    // The whole record has to be there before the old one's stores are issued:
+    // loads and stores complete in order, so any later wait for the loads
+    // would be one for the stores too.
+    asm volatile("" ::"v"(hb.lnw), "v"(hb.hist), "v"(cb.etot), "v"(cb.esq), "v"(cb.rt), "v"(cb.vep), "v"(wl2));
+    const double w2 = same ? c_lnw : hb.lnw, l2 = ext2 ? out2 : w2;
     const uint64_t h2 = same ? c_hist : hb.hist;
-    const bool acc = !reject_move(go, e1, e2, w2, h2) && go;
+    const bool acc = go & !reject_move(go, e1, e2, l1, l2, h2);
     accepted += acc ? 1 : 0;
     acc_rate = acc ? acc_rate + rs : acc_rate;
-    if (acc) {
-      confirm();
-      int32_t i = i2;
-      if (__builtin_expect(E != e2, 0)) i = e_index(E);
-      if (__builtin_expect(i != i2, 0)) {
-        if (idx_ok(i) && base + i != cur_p) load_current(base + i);
-      } else if (!same) {
-        set_current(p2, hb, cb, wl2);
-      }
+    const bool trip = take_energy(acc, e2, pdabse);
+    if (acc) confirm_system();
+    if (acc & !same) set_current(p2, hb, cb, wl2);
+    cur_i = acc ? i2 : cur_i;
+    return trip;
+  }
+  // After a recomputed energy, which may lie in another bin.
+  SADMC_DF void reindex() {
+    const int32_t i = e_index(E);
+    if (i != cur_i && idx_ok(i)) {
+      load_current(base + i);
       cur_i = i;
     }
-    if (__builtin_expect(status == 0, 1)) visit(i1);
   }
-  SADMC_DF void visit(int32_t i1) {
+  // The update of the bin the walker is in.
+  SADMC_DF void visit() {
+    const int32_t i1 = from_i;
     const double En = E;
     const int32_t i = cur_i;
     const int32_t p = cur_p;
     if (__builtin_expect(c_hist == 0, 0)) {
       tfound()[p] = moves();
-      if (METH == M_SAD && i >= ilo && i <= ihi) rec().tmax = moves();
+      if (METH == M_SAD && i >= ilo && i <= ihi) tmax = tm;
     }
     c_hist += 1;
     if (SYS == SYS_WCA && args().collect_pressure && __builtin_expect(tm == next_press, 0)) {
@@ -1339,7 +1519,7 @@ struct Engine {
     // energy.rs:950-965 and 941-943 (the energy of this move's end is added
     // at the start of the next in the reference; nothing between reads it)
     bool round_trip = true;
-    if (__builtin_expect(c_lnw > max_S || i == max_S_index, 0)) {
+    if (__builtin_expect((c_lnw > max_S) | (i == max_S_index), 0)) {
       round_trip = false;
       if (c_lnw > max_S) {
         max_S = c_lnw;
@@ -1351,12 +1531,20 @@ struct Engine {
         bulk = 0;
       }
     }
-    if (round_trip && !(bulk || c_vep == epoch)) {
-      c_vep = epoch;
-      c_rt += 1;
-    }
+    const bool mark = round_trip & !((bulk != 0) | (c_vep == epoch));
+    c_vep = mark ? epoch : c_vep;
+    c_rt += mark ? 1 : 0;
     c_etot += En;
     c_esq += En * En;
+  }
+
+  // rs_wave for the next 64 moves: what every walker needs each move, from one
+  // square root per lane.
+  SADMC_DF void next_roots() {
+    const uint64_t on = __ballot(status == 0);
+    const double t = __shfl(tm, (int)__builtin_ctzll(on), 64);
+    rs_same = __ballot(1) == ~0ULL && !__any((status == 0) & (tm != t));
+    rs_wave = sqrt(1.0 / (t + (double)((threadIdx.x & 63) + 1)));
   }
 
   SADMC_DF void run(uint64_t nmoves) {
@@ -1364,7 +1552,18 @@ struct Engine {
     // the compiler keep the state of stopped and running walkers apart, which
     // took 80 more registers)
     for (uint64_t k = 0; k < nmoves && __any(status == 0); k++) {
-      if (__builtin_expect(status == 0, 1)) move_once();
+      const int step = (int)(k & 63);
+      if (step == 0) next_roots();
+      bool trip = false;
+      if (__builtin_expect(status == 0, 1)) trip = propose(step);
+      if (__builtin_expect(__any(trip), 0)) {
+        full_energies(trip);
+        if (trip) {
+          took_full_energy();
+          reindex();
+        }
+      }
+      if (__builtin_expect(status == 0, 1)) visit();
     }
   }
 

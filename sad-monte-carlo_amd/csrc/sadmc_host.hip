@@ -64,7 +64,7 @@ struct SetHost {
   uint64_t *d_spins = nullptr;
   HotBin *d_hot = nullptr;
   ColdBin *d_cold = nullptr;
-  uint64_t *d_tf = nullptr;
+  uint64_t *d_tf = nullptr;  // part of d_cold's allocation
   uint64_t *d_wlh = nullptr;
   PExtra *d_extra = nullptr;
   Pending *d_pending = nullptr;
@@ -375,7 +375,6 @@ static void free_set(SetHost &s) {
   (void)hipFree(s.d_spins);
   (void)hipFree(s.d_hot);
   (void)hipFree(s.d_cold);
-  (void)hipFree(s.d_tf);
   (void)hipFree(s.d_wlh);
   (void)hipFree(s.d_extra);
   (void)hipFree(s.d_pending);
@@ -537,6 +536,8 @@ static void fill_args(SetHost &s) {
   a.move_param = s.p.move_param;
   a.min_e = s.p.min_e;
   a.max_e = s.p.max_e;
+  a.floor_e = s.p.has_min_e ? s.p.min_e : -INFINITY;
+  a.ceil_e = s.p.has_max_e ? s.p.max_e : INFINITY;
   a.rc2 = s.p.rc2;
   a.width = s.width;
   a.inv_width = 1.0 / s.width;
@@ -630,10 +631,10 @@ int sadmc_init(sadmc_ctx *c) {
     const size_t nb = (size_t)W * s.cap;
     HIPCHECK(c, hipMalloc(&s.d_hot, sizeof(HotBin) * nb));
     HIPCHECK(c, hipMemsetAsync(s.d_hot, 0, sizeof(HotBin) * nb, c->stream));
-    HIPCHECK(c, hipMalloc(&s.d_cold, sizeof(ColdBin) * nb));
-    HIPCHECK(c, hipMemsetAsync(s.d_cold, 0, sizeof(ColdBin) * nb, c->stream));
-    HIPCHECK(c, hipMalloc(&s.d_tf, sizeof(uint64_t) * nb));
-    HIPCHECK(c, hipMemsetAsync(s.d_tf, 0, sizeof(uint64_t) * nb, c->stream));
+    // the cold records and, behind them, t_found
+    HIPCHECK(c, hipMalloc(&s.d_cold, (sizeof(ColdBin) + sizeof(uint64_t)) * nb));
+    HIPCHECK(c, hipMemsetAsync(s.d_cold, 0, (sizeof(ColdBin) + sizeof(uint64_t)) * nb, c->stream));
+    s.d_tf = (uint64_t *)(s.d_cold + nb);
     if (s.p.method == SADMC_WL || s.p.method == SADMC_INV_T_WL) {
       HIPCHECK(c, hipMalloc(&s.d_wlh, sizeof(uint64_t) * nb));
       HIPCHECK(c, hipMemsetAsync(s.d_wlh, 0, sizeof(uint64_t) * nb, c->stream));

@@ -139,20 +139,40 @@ hipError_t launch_pt(int sys, int kmax, const SetArgs &a, const PtArgs &p, int l
 
 #ifdef SADMC_KERNEL_TU
 
-// GC > 0: the set's lanes per walker as a compile-time constant.  A
-// workgroup of one to four wavefronts holds blockDim.x / G walkers.
+// Walkers per wavefront of the run kernel: as many as fit (64 / G), unless
+// that leaves SIMDs without a wave; then half as many, and so on down to one.
+// A wave takes the branches that any of its walkers takes and waits for all
+// their records, so fewer walkers per wave cost less per move as long as each
+// wave has a SIMD to itself (1024 of them): 4096 LJ13 walkers take 2.09 us a
+// move at 4 walkers a wave, 2.50 at 16 and 2.85 at 2.  The Ising walker's chain
+// is short enough that two waves share a SIMD without loss: 4096 walkers take
+// 1.91 us a move at 2 a wave, 2.19 at 4, 2.41 at 64 and 3.4 at 1.
+static inline int walkers_per_wave(int W, int G) {
+  const int target = G == 1 ? 2048 : 1024;
+  int per = 64 / G;
+  while (per > 1 && (W + per - 1) / per < target) per /= 2;
+  return per;
+}
+
+// GC > 0: the set's lanes per walker as a compile-time constant.  Each of a
+// workgroup's one to four wavefronts holds `per` walkers, 64/G or fewer.
 template <int SYS, int KMAX, int PREC, int METH, int GC = 0>
-__global__ __launch_bounds__(256) void k_run(SetArgs a, uint64_t moves) {
+__global__ __launch_bounds__(256) void k_run(SetArgs a, uint64_t moves, int per) {
   extern __shared__ double lds[];
   const int G = GC ? GC : a.G;
-  const int group = threadIdx.x / G;
+  const int wave = threadIdx.x / 64, group = (threadIdx.x & 63) / G;
   const int lane = threadIdx.x & (G - 1);
-  const int walker = blockIdx.x * (blockDim.x / G) + group;
-  if (walker >= a.W) return;
+  const int walker = (blockIdx.x * (blockDim.x / 64) + wave) * per + group;
+  double *tile = lds + (wave * per + group) * 3 * a.npad;
   Engine<SYS, KMAX, PREC, METH, 0, GC> e;
-  e.load(a, walker, lane, lds + group * 3 * a.npad);
+  const bool held = group < per && walker < a.W;
+  if (held) {
+    e.load(a, walker, lane, tile);
+  } else {
+    e.load_idle(a, lane, tile);
+  }
   e.run(moves);
-  e.store(walker);
+  if (held) e.store(walker);
 }
 
 template <int SYS, int KMAX, int PREC, int METH>
@@ -215,13 +235,17 @@ __global__ __launch_bounds__(64) void k_confirm(SetArgs a, int walker, const Pen
 template <int SYS, int KMAX, int PREC, int METH>
 __global__ __launch_bounds__(64) void k_energy(SetArgs a, int walker, double *out) {
   extern __shared__ double lds[];
-  if ((int)threadIdx.x >= a.G) return;
+  const bool held = (int)threadIdx.x < a.G;
   Engine<SYS, KMAX, PREC, METH> e;
-  e.load_system(a, walker, threadIdx.x, lds);
-  e.L = a.ws[walker].geom;
-  e.halfL = 0.5 * e.L;
-  const double en = e.full_energy();
-  if (threadIdx.x == 0) *out = en;
+  if (held) {
+    e.load_system(a, walker, threadIdx.x, lds);
+    e.L = a.ws[walker].geom;
+    e.halfL = 0.5 * e.L;
+  } else {
+    e.load_idle(a, threadIdx.x & (a.G - 1), lds + threadIdx.x / a.G * 3 * a.npad);
+  }
+  e.full_energies(held);
+  if (threadIdx.x == 0) *out = e.E;
 }
 
 template <int SYS, int KMAX, int PREC, int METH>
@@ -233,7 +257,8 @@ static hipError_t launch_t(KernelKind kk, const SetArgs &a, const LaunchArgs &la
   const dim3 grid((a.W + per_block - 1) / per_block), block(64);
   // the run kernel: la.waves wavefronts per workgroup
   const int wv = la.waves > 1 ? la.waves : 1;
-  const int run_per_block = wv * per_block;
+  const int per = walkers_per_wave(a.W, G);
+  const int run_per_block = wv * per;
   const size_t run_lds = SYS == SYS_ISING ? 0 : (size_t)run_per_block * 3 * a.npad * sizeof(double);
   const dim3 run_grid((a.W + run_per_block - 1) / run_per_block), run_block(64 * wv);
   switch (kk) {
@@ -242,19 +267,22 @@ static hipError_t launch_t(KernelKind kk, const SetArgs &a, const LaunchArgs &la
       // the lanes fixed at compile time
       if constexpr (SYS != SYS_ISING && METH == M_SAD && KMAX >= 2 && KMAX <= 8) {
         if (a.G == 4) {
-          hipLaunchKernelGGL((k_run<SYS, KMAX, PREC, METH, 4>), run_grid, run_block, run_lds, s, a, la.moves);
+          hipLaunchKernelGGL((k_run<SYS, KMAX, PREC, METH, 4>), run_grid, run_block, run_lds, s, a, la.moves,
+                             per);
           break;
         }
         if (a.G == 8) {
-          hipLaunchKernelGGL((k_run<SYS, KMAX, PREC, METH, 8>), run_grid, run_block, run_lds, s, a, la.moves);
+          hipLaunchKernelGGL((k_run<SYS, KMAX, PREC, METH, 8>), run_grid, run_block, run_lds, s, a, la.moves,
+                             per);
           break;
         }
         if (a.G == 16) {
-          hipLaunchKernelGGL((k_run<SYS, KMAX, PREC, METH, 16>), run_grid, run_block, run_lds, s, a, la.moves);
+          hipLaunchKernelGGL((k_run<SYS, KMAX, PREC, METH, 16>), run_grid, run_block, run_lds, s, a, la.moves,
+                             per);
           break;
         }
       }
-      hipLaunchKernelGGL((k_run<SYS, KMAX, PREC, METH>), run_grid, run_block, run_lds, s, a, la.moves);
+      hipLaunchKernelGGL((k_run<SYS, KMAX, PREC, METH>), run_grid, run_block, run_lds, s, a, la.moves, per);
       break;
     case KK_INIT:
       hipLaunchKernelGGL((k_init<SYS, KMAX, PREC, METH>), grid, block, lds, s, a, la.e_lo);
