@@ -94,3 +94,22 @@ def test_energy_query_is_the_lane_group_sum(gpu_ctx_factory, kw, geom):
                 part = part[0::2] + part[1::2]
             want = float(part[0])
         assert ctx.compute_energy(s, w) == want
+
+
+@pytest.mark.parametrize("binning", [S.BIN_HISTOGRAM, S.BIN_LINEAR])
+@pytest.mark.parametrize("kw,geom,sizes", [
+    pytest.param(LJ13, 2.5, (3, 2049, 17000), id="lj13"),
+    pytest.param(dict(WCA32, method=S.WL, method_param=1e-6), 4.2, (3, 8195), id="wca32-wl"),
+    pytest.param(ISING, None, (3, 5000, 131100), id="ising"),
+])
+def test_binning_walkers_do_not_depend_on_their_wave(gpu_ctx_factory, kw, geom, sizes, binning):
+    ref = None
+    for walkers in sizes:
+        ctx = gpu_ctx_factory()
+        s = ctx.bin_add_set(S.make_params(binning=binning, **kw), np.arange(walkers, dtype=np.uint64) + 11, geom=geom)
+        ctx.bin_run(s, 700)
+        ctx.bin_run(s, 500)
+        got = [(ctx.bin_state(s, w).tobytes(), ctx.bin_bins(s, w).tobytes()) for w in range(sizes[0])]
+        ctx.close()
+        ref = ref or got
+        assert got == ref, f"{walkers} walkers"
