@@ -4,6 +4,7 @@
 
 #include <algorithm>
 #include <map>
+#include <mutex>
 #include <cmath>
 #include <cstdio>
 #include <cstring>
@@ -69,7 +70,6 @@ struct SetHost {
   PExtra *d_extra = nullptr;
   Pending *d_pending = nullptr;
   int32_t *d_flag = nullptr;
-  double *d_eout = nullptr;  // a recomputed energy (sadmc_compute_energy)
   int waves = 1;             // wavefronts per workgroup of the run kernel
   SetArgs args;
 };
@@ -158,6 +158,12 @@ struct sadmc_ctx {
   // entropy reduction scratch, grown on demand and kept for later calls
   void *d_ent = nullptr;
   size_t ent_bytes = 0;
+  // the walker sets' stop flags, one each, so that a sync reads them at once
+  int32_t *d_flags = nullptr;
+  // pinned staging for small reads (kPinBytes, made on first use); one reader
+  // at a time
+  char *pin = nullptr;
+  std::mutex pin_mu;
 };
 
 static int fail(sadmc_ctx *c, int code, const std::string &msg) {
@@ -194,6 +200,29 @@ struct AllocGuard {
 // LJ initial positions (uniform in the sphere, all pairs >= 0.8 sigma):
 // atoms are added one at a time, each drawn by rejection from [-R, R)^3 and
 // redrawn until it is inside the sphere and 0.8 sigma from every earlier atom.
+// Small reads go through pinned memory: a copy to pageable memory costs the
+// runtime its own staging and a blocking wait (a walker's record: 45 us a
+// call; 13 us this way).
+constexpr size_t kPinBytes = 1 << 16;
+static hipError_t staging(sadmc_ctx *c) {  // under pin_mu
+  return c->pin ? hipSuccess : hipHostMalloc((void **)&c->pin, kPinBytes, hipHostMallocDefault);
+}
+
+// `bytes` at the device address `src` into `dst`, after everything queued on
+// the context's stream.
+static hipError_t fetch(sadmc_ctx *c, void *dst, const void *src, size_t bytes) {
+  if (bytes > kPinBytes) {
+    const hipError_t e = hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, c->stream);
+    return e != hipSuccess ? e : hipStreamSynchronize(c->stream);
+  }
+  std::lock_guard<std::mutex> hold(c->pin_mu);
+  hipError_t e = staging(c);
+  if (e == hipSuccess) e = hipMemcpyAsync(c->pin, src, bytes, hipMemcpyDeviceToHost, c->stream);
+  if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
+  if (e == hipSuccess) std::memcpy(dst, c->pin, bytes);
+  return e;
+}
+
 static int lj_init_coords(int n, double radius, uint64_t seed, double *c) {
   uint64_t s0, s1;
   rng_seed(seed ^ kInitTag, s0, s1);
@@ -292,10 +321,10 @@ static int gather_bins(sadmc_ctx *c, const SetHost &s, int w, int64_t first, int
   std::vector<ColdBin> cb(count);
   std::vector<uint64_t> tf(count), wl(count, 0);
   const size_t off = (size_t)w * s.cap + first;
-  HIPCHECK(c, hipMemcpy(h.data(), s.d_hot + off, sizeof(HotBin) * count, hipMemcpyDeviceToHost));
-  HIPCHECK(c, hipMemcpy(cb.data(), s.d_cold + off, sizeof(ColdBin) * count, hipMemcpyDeviceToHost));
-  HIPCHECK(c, hipMemcpy(tf.data(), s.d_tf + off, sizeof(uint64_t) * count, hipMemcpyDeviceToHost));
-  if (s.d_wlh) HIPCHECK(c, hipMemcpy(wl.data(), s.d_wlh + off, sizeof(uint64_t) * count, hipMemcpyDeviceToHost));
+  HIPCHECK(c, fetch(c, h.data(), s.d_hot + off, sizeof(HotBin) * count));
+  HIPCHECK(c, fetch(c, cb.data(), s.d_cold + off, sizeof(ColdBin) * count));
+  HIPCHECK(c, fetch(c, tf.data(), s.d_tf + off, sizeof(uint64_t) * count));
+  if (s.d_wlh) HIPCHECK(c, fetch(c, wl.data(), s.d_wlh + off, sizeof(uint64_t) * count));
   for (int64_t k = 0; k < count; k++) {
     out[k].lnw = h[k].lnw;
     out[k].histogram = h[k].hist;
@@ -378,9 +407,6 @@ static void free_set(SetHost &s) {
   (void)hipFree(s.d_wlh);
   (void)hipFree(s.d_extra);
   (void)hipFree(s.d_pending);
-  (void)hipFree(s.d_flag);
-  (void)hipFree(s.d_eout);
-  s.d_eout = nullptr;
   s.d_ws = nullptr;
   s.d_pos = nullptr;
   s.d_spins = nullptr;
@@ -406,6 +432,8 @@ void sadmc_destroy(sadmc_ctx *c) {
                   (void *)c->d_partial, (void *)c->d_grad, (void *)c->d_loss})
     (void)hipFree(p);
   (void)hipFree(c->d_ent);
+  (void)hipFree(c->d_flags);
+  if (c->pin) (void)hipHostFree(c->pin);
   for (auto &z : c->zmcs)
     for (void *p : {(void *)z.d_sim, (void *)z.d_rep, (void *)z.d_slot, (void *)z.d_med, (void *)z.d_pos,
                     (void *)z.d_geom, (void *)z.d_slot_of, (void *)z.d_spins})
@@ -549,11 +577,13 @@ static void fill_args(SetHost &s) {
 }
 
 static int check_flags(sadmc_ctx *c) {
+  if (c->sets.empty()) return SADMC_OK;
+  if (!c->d_flags) return fail(c, SADMC_E_HIP, "the walker sets hold no device memory yet");
+  std::vector<int32_t> flags(c->sets.size());
+  HIPCHECK(c, fetch(c, flags.data(), c->d_flags, sizeof(int32_t) * flags.size()));
   for (size_t k = 0; k < c->sets.size(); k++) {
     SetHost &s = c->sets[k];
-    int32_t flag = 0;
-    HIPCHECK(c, hipMemcpy(&flag, s.d_flag, sizeof(int32_t), hipMemcpyDeviceToHost));
-    if (!flag) continue;
+    if (!flags[k]) continue;
     std::vector<sadmc_walker_state> ws(s.W);
     HIPCHECK(c, hipMemcpy(ws.data(), s.d_ws, sizeof(sadmc_walker_state) * s.W, hipMemcpyDeviceToHost));
     for (int w = 0; w < s.W; w++) {
@@ -625,6 +655,9 @@ int sadmc_init(sadmc_ctx *c) {
   if (c->inited) return fail(c, SADMC_E_STATE, "already initialised");
   if (c->sets.empty()) return fail(c, SADMC_E_STATE, "no walker sets");
   HIPCHECK(c, hipSetDevice(c->device));
+  const size_t flag_bytes = sizeof(int32_t) * c->sets.size();
+  if (!c->d_flags) HIPCHECK(c, hipMalloc(&c->d_flags, flag_bytes));
+  HIPCHECK(c, hipMemsetAsync(c->d_flags, 0, flag_bytes, c->stream));
   for (auto &s : c->sets) {
     const int W = s.W, n = s.p.n;
     HIPCHECK(c, hipMalloc(&s.d_ws, sizeof(sadmc_walker_state) * W));
@@ -640,9 +673,7 @@ int sadmc_init(sadmc_ctx *c) {
       HIPCHECK(c, hipMemsetAsync(s.d_wlh, 0, sizeof(uint64_t) * nb, c->stream));
     }
     HIPCHECK(c, hipMalloc(&s.d_pending, sizeof(Pending)));
-    HIPCHECK(c, hipMalloc(&s.d_eout, sizeof(double)));
-    HIPCHECK(c, hipMalloc(&s.d_flag, sizeof(int32_t)));
-    HIPCHECK(c, hipMemsetAsync(s.d_flag, 0, sizeof(int32_t), c->stream));
+    s.d_flag = c->d_flags + (&s - c->sets.data());
     std::vector<sadmc_walker_state> ws(W);
     std::memset(ws.data(), 0, sizeof(sadmc_walker_state) * W);
     for (int w = 0; w < W; w++) {
@@ -769,8 +800,8 @@ int sadmc_check_recip_f32(int device, int32_t what, uint64_t lo, uint64_t hi, ui
 
 int sadmc_sync(sadmc_ctx *c) {
   if (!c) return SADMC_E_ARG;
-  HIPCHECK(c, hipStreamSynchronize(c->stream));
-  return check_flags(c);
+  if (c->sets.empty() || !c->d_flags) HIPCHECK(c, hipStreamSynchronize(c->stream));
+  return check_flags(c);  // (reads the flags after everything on the stream)
 }
 
 int sadmc_last_run_ms(const sadmc_ctx *c, double *ms) {
@@ -1038,8 +1069,7 @@ int sadmc_plan_move(sadmc_ctx *c, int32_t set, int32_t walker, double scale, dou
   la.pending = s->d_pending;
   HIPCHECK(c, launch(s->p.system, s->p.precision, s->p.method, s->KMAX, KK_PLAN, s->args, la, c->stream));
   Pending p;
-  HIPCHECK(c, hipMemcpyAsync(&p, s->d_pending, sizeof p, hipMemcpyDeviceToHost, c->stream));
-  HIPCHECK(c, hipStreamSynchronize(c->stream));
+  HIPCHECK(c, fetch(c, &p, s->d_pending, sizeof p));
   if (e_new) *e_new = p.e;
   if (some) *some = p.some;
   return SADMC_OK;
@@ -1068,8 +1098,7 @@ int sadmc_plan_learned(sadmc_ctx *c, int32_t set, int32_t walker, double *e_new,
   la.pending = s->d_pending;
   HIPCHECK(c, launch(s->p.system, s->p.precision, s->p.method, s->KMAX, KK_PLAN, s->args, la, c->stream));
   Pending p;
-  HIPCHECK(c, hipMemcpyAsync(&p, s->d_pending, sizeof p, hipMemcpyDeviceToHost, c->stream));
-  HIPCHECK(c, hipStreamSynchronize(c->stream));
+  HIPCHECK(c, fetch(c, &p, s->d_pending, sizeof p));
   if (e_new) *e_new = p.e;
   if (lnh) *lnh = p.dabse;
   if (to) {
@@ -1218,8 +1247,7 @@ int sadmc_prop_train(sadmc_ctx *c, int32_t steps, int32_t batch, float lr, float
                                    c->prop_step, nullptr, c->d_loss + k, c->stream));
   }
   if (losses)
-    HIPCHECK(c, hipMemcpyAsync(losses, c->d_loss, sizeof(float) * steps, hipMemcpyDeviceToHost, c->stream));
-  HIPCHECK(c, hipStreamSynchronize(c->stream));
+    HIPCHECK(c, fetch(c, losses, c->d_loss, sizeof(float) * steps));
   return SADMC_OK;
 }
 
@@ -1276,8 +1304,12 @@ int mean_entropy_impl(sadmc_ctx *c, int32_t set, double e_a, double e_b, int64_t
   if (!base) return fixed_base ? SADMC_E_CAPACITY : SADMC_E_HIP;
   EntropyRange range;
   HIPCHECK(c, launch_entropy_range(s->d_ws, s->W, w, (EntropyRange *)base, (EntropyRange *)base + 1, c->stream));
-  HIPCHECK(c, hipMemcpyAsync(&range, base, sizeof range, hipMemcpyDeviceToHost, c->stream));
-  HIPCHECK(c, hipStreamSynchronize(c->stream));
+  if (fixed_base) {  // no allocation: not even the staging buffer
+    HIPCHECK(c, hipMemcpyAsync(&range, base, sizeof range, hipMemcpyDeviceToHost, c->stream));
+    HIPCHECK(c, hipStreamSynchronize(c->stream));
+  } else {
+    HIPCHECK(c, fetch(c, &range, base, sizeof range));
+  }
   if (!range.any) return fail(c, SADMC_E_STATE, "no running walkers");
   const double gmin = range.gmin;
   const int64_t ng = range.ng;
@@ -1324,10 +1356,13 @@ int sadmc_compute_energy(sadmc_ctx *c, int32_t set, int32_t walker, double *e) {
   HIPCHECK(c, hipSetDevice(c->device));
   LaunchArgs la{};
   la.walker = walker;
-  la.eout = s->d_eout;
+  // the kernel writes the energy straight into pinned memory
+  std::lock_guard<std::mutex> hold(c->pin_mu);
+  HIPCHECK(c, staging(c));
+  la.eout = (double *)c->pin;
   HIPCHECK(c, launch(s->p.system, s->p.precision, s->p.method, s->KMAX, KK_ENERGY, s->args, la, c->stream));
-  HIPCHECK(c, hipMemcpyAsync(e, s->d_eout, sizeof(double), hipMemcpyDeviceToHost, c->stream));
   HIPCHECK(c, hipStreamSynchronize(c->stream));
+  *e = *(volatile double *)c->pin;
   return SADMC_OK;
 }
 
@@ -1409,8 +1444,7 @@ int sadmc_walker_count(const sadmc_ctx *c, int32_t set, int32_t *n, int64_t *cap
 int sadmc_get_walker_state(sadmc_ctx *c, int32_t set, int32_t walker, sadmc_walker_state *out) {
   SetHost *s = get_set(c, set, walker);
   if (!s || !out || !c->inited) return fail(c, SADMC_E_ARG, "bad set/walker or not initialised");
-  HIPCHECK(c, hipStreamSynchronize(c->stream));
-  HIPCHECK(c, hipMemcpy(out, s->d_ws + walker, sizeof *out, hipMemcpyDeviceToHost));
+  HIPCHECK(c, fetch(c, out, s->d_ws + walker, sizeof *out));
   return SADMC_OK;
 }
 
@@ -1431,8 +1465,7 @@ int sadmc_walker_bins(sadmc_ctx *c, int32_t set, int32_t walker, int64_t cap, do
   std::vector<PExtra> x;
   if (s->d_extra) {
     x.resize(st.len);
-    HIPCHECK(c, hipMemcpy(x.data(), s->d_extra + (size_t)walker * s->cap + st.base, sizeof(PExtra) * st.len,
-                          hipMemcpyDeviceToHost));
+    HIPCHECK(c, fetch(c, x.data(), s->d_extra + (size_t)walker * s->cap + st.base, sizeof(PExtra) * st.len));
   }
   for (int64_t i = 0; i < st.len; i++) {
     if (lnw) lnw[i] = b[i].lnw;
@@ -1453,9 +1486,7 @@ int sadmc_walker_coords(sadmc_ctx *c, int32_t set, int32_t walker, double *coord
   SetHost *s = get_set(c, set, walker);
   if (!s || !coords || !c->inited || s->p.system == SADMC_ISING) return fail(c, SADMC_E_ARG, "bad arguments");
   std::vector<double> p((size_t)3 * s->npad);
-  HIPCHECK(c, hipStreamSynchronize(c->stream));
-  HIPCHECK(c, hipMemcpy(p.data(), s->d_pos + (size_t)walker * 3 * s->npad, sizeof(double) * p.size(),
-                        hipMemcpyDeviceToHost));
+  HIPCHECK(c, fetch(c, p.data(), s->d_pos + (size_t)walker * 3 * s->npad, sizeof(double) * p.size()));
   const int n = s->p.n;
   for (int d = 0; d < 3; d++)
     for (int j = 0; j < n; j++) coords[d * n + j] = p[(size_t)d * s->npad + j];
@@ -1466,8 +1497,7 @@ int sadmc_walker_spins(sadmc_ctx *c, int32_t set, int32_t walker, int8_t *spins)
   SetHost *s = get_set(c, set, walker);
   if (!s || !spins || !c->inited || s->p.system != SADMC_ISING) return fail(c, SADMC_E_ARG, "bad arguments");
   uint64_t bits = 0;
-  HIPCHECK(c, hipStreamSynchronize(c->stream));
-  HIPCHECK(c, hipMemcpy(&bits, s->d_spins + walker, sizeof bits, hipMemcpyDeviceToHost));
+  HIPCHECK(c, fetch(c, &bits, s->d_spins + walker, sizeof bits));
   const int n = s->p.n;
   for (int b = 0; b < n * n; b++) spins[b] = ((bits >> b) & 1ULL) ? 1 : -1;
   return SADMC_OK;
@@ -1698,16 +1728,14 @@ int sadmc_pt_run(sadmc_ctx *c, int32_t pt, uint64_t rounds) {
 int sadmc_pt_replicas(sadmc_ctx *c, int32_t pt, sadmc_replica *out) {
   PtHost *t = pt_get(c, pt);
   if (!t || !out) return fail(c, SADMC_E_ARG, "no such tempering ladder set or null output");
-  HIPCHECK(c, hipMemcpyAsync(out, t->d_rep, sizeof(sadmc_replica) * t->L * t->R, hipMemcpyDeviceToHost, c->stream));
-  HIPCHECK(c, hipStreamSynchronize(c->stream));
+  HIPCHECK(c, fetch(c, out, t->d_rep, sizeof(sadmc_replica) * t->L * t->R));
   return SADMC_OK;
 }
 
 static int pt_slot(sadmc_ctx *c, PtHost *t, int32_t l, int32_t r, int64_t *slot) {
   if (l < 0 || l >= t->L || r < 0 || r >= t->R) return fail(c, SADMC_E_ARG, "ladder or replica out of range");
   int32_t s = 0;
-  HIPCHECK(c, hipMemcpyAsync(&s, t->d_slot_of + (int64_t)l * t->R + r, sizeof s, hipMemcpyDeviceToHost, c->stream));
-  HIPCHECK(c, hipStreamSynchronize(c->stream));
+  HIPCHECK(c, fetch(c, &s, t->d_slot_of + (int64_t)l * t->R + r, sizeof s));
   *slot = (int64_t)l * t->R + s;
   return SADMC_OK;
 }
@@ -1720,10 +1748,10 @@ int sadmc_pt_coords(sadmc_ctx *c, int32_t pt, int32_t l, int32_t r, double *coor
   int rc = pt_slot(c, t, l, r, &slot);
   if (rc) return rc;
   const int n = t->args.n;
+  std::vector<double> p((size_t)3 * t->npad);
+  HIPCHECK(c, fetch(c, p.data(), t->d_pos + slot * 3 * t->npad, sizeof(double) * p.size()));
   for (int d = 0; d < 3; d++)
-    HIPCHECK(c, hipMemcpyAsync(coords + (size_t)d * n, t->d_pos + (slot * 3 + d) * t->npad, sizeof(double) * n,
-                               hipMemcpyDeviceToHost, c->stream));
-  HIPCHECK(c, hipStreamSynchronize(c->stream));
+    for (int j = 0; j < n; j++) coords[d * n + j] = p[(size_t)d * t->npad + j];
   return SADMC_OK;
 }
 
@@ -1735,8 +1763,7 @@ int sadmc_pt_spins(sadmc_ctx *c, int32_t pt, int32_t l, int32_t r, int8_t *spins
   int rc = pt_slot(c, t, l, r, &slot);
   if (rc) return rc;
   uint64_t b = 0;
-  HIPCHECK(c, hipMemcpyAsync(&b, t->d_spins + slot, sizeof b, hipMemcpyDeviceToHost, c->stream));
-  HIPCHECK(c, hipStreamSynchronize(c->stream));
+  HIPCHECK(c, fetch(c, &b, t->d_spins + slot, sizeof b));
   const int n = t->args.n;
   for (int k = 0; k < n * n; k++) spins[k] = ((b >> k) & 1ULL) ? 1 : -1;
   return SADMC_OK;
@@ -1745,8 +1772,7 @@ int sadmc_pt_spins(sadmc_ctx *c, int32_t pt, int32_t l, int32_t r, int8_t *spins
 int sadmc_pt_ladder_rng(sadmc_ctx *c, int32_t pt, uint64_t *out) {
   PtHost *t = pt_get(c, pt);
   if (!t || !out) return fail(c, SADMC_E_ARG, "no such tempering ladder set or null output");
-  HIPCHECK(c, hipMemcpyAsync(out, t->d_lrng, sizeof(uint64_t) * 2 * t->L, hipMemcpyDeviceToHost, c->stream));
-  HIPCHECK(c, hipStreamSynchronize(c->stream));
+  HIPCHECK(c, fetch(c, out, t->d_lrng, sizeof(uint64_t) * 2 * t->L));
   return SADMC_OK;
 }
 
@@ -1922,8 +1948,7 @@ int sadmc_bin_run(sadmc_ctx *c, int32_t set, uint64_t moves) {
     c->timed = true;
   }
   int32_t flag = 0;
-  HIPCHECK(c, hipMemcpyAsync(&flag, b->d_flag, sizeof flag, hipMemcpyDeviceToHost, c->stream));
-  HIPCHECK(c, hipStreamSynchronize(c->stream));
+  HIPCHECK(c, fetch(c, &flag, b->d_flag, sizeof flag));
   if (!flag) return SADMC_OK;
   std::vector<sadmc_bwalker_state> ws(b->W);
   HIPCHECK(c, hipMemcpy(ws.data(), b->d_ws, sizeof(sadmc_bwalker_state) * b->W, hipMemcpyDeviceToHost));
@@ -1942,8 +1967,7 @@ int sadmc_bin_run(sadmc_ctx *c, int32_t set, uint64_t moves) {
 int sadmc_bin_state(sadmc_ctx *c, int32_t set, int32_t w, sadmc_bwalker_state *out) {
   BinSetHost *b = bset_get(c, set);
   if (!b || !out || w < 0 || w >= b->W) return fail(c, SADMC_E_ARG, "no such binning walker or null output");
-  HIPCHECK(c, hipMemcpyAsync(out, b->d_ws + w, sizeof *out, hipMemcpyDeviceToHost, c->stream));
-  HIPCHECK(c, hipStreamSynchronize(c->stream));
+  HIPCHECK(c, fetch(c, out, b->d_ws + w, sizeof *out));
   return SADMC_OK;
 }
 
@@ -1954,9 +1978,7 @@ int sadmc_bin_bins(sadmc_ctx *c, int32_t set, int32_t w, int64_t max_bins, sadmc
   if (st.len > max_bins || !out) return fail(c, SADMC_E_CAPACITY, "output holds fewer bins than the walker has");
   BinSetHost *b = bset_get(c, set);
   if (st.len > 0)
-    HIPCHECK(c, hipMemcpyAsync(out, b->d_bins + (int64_t)w * b->cap + st.base, sizeof(sadmc_bbin) * st.len,
-                               hipMemcpyDeviceToHost, c->stream));
-  HIPCHECK(c, hipStreamSynchronize(c->stream));
+    HIPCHECK(c, fetch(c, out, b->d_bins + (int64_t)w * b->cap + st.base, sizeof(sadmc_bbin) * st.len));
   return SADMC_OK;
 }
 
@@ -1964,14 +1986,11 @@ int sadmc_bin_hires(sadmc_ctx *c, int32_t set, int32_t w, sadmc_hires *out, int6
   BinSetHost *b = bset_get(c, set);
   if (!b || !out || w < 0 || w >= b->W) return fail(c, SADMC_E_ARG, "no such binning walker or null output");
   if (!b->hr_cap) return fail(c, SADMC_E_ARG, "the set keeps no high_resolution histogram");
-  HIPCHECK(c, hipMemcpyAsync(out, b->d_hrs + w, sizeof *out, hipMemcpyDeviceToHost, c->stream));
-  HIPCHECK(c, hipStreamSynchronize(c->stream));
+  HIPCHECK(c, fetch(c, out, b->d_hrs + w, sizeof *out));
   if (!counts) return SADMC_OK;
   if (out->len > max_bins) return fail(c, SADMC_E_CAPACITY, "output holds fewer bins than the side histogram has");
   if (out->len > 0)
-    HIPCHECK(c, hipMemcpyAsync(counts, b->d_hr + (int64_t)w * b->hr_cap + out->base, sizeof(uint64_t) * out->len,
-                               hipMemcpyDeviceToHost, c->stream));
-  HIPCHECK(c, hipStreamSynchronize(c->stream));
+    HIPCHECK(c, fetch(c, counts, b->d_hr + (int64_t)w * b->hr_cap + out->base, sizeof(uint64_t) * out->len));
   return SADMC_OK;
 }
 
@@ -1980,10 +1999,10 @@ int sadmc_bin_coords(sadmc_ctx *c, int32_t set, int32_t w, double *coords) {
   if (!b || !coords || w < 0 || w >= b->W) return fail(c, SADMC_E_ARG, "no such binning walker or null output");
   if (b->sys == SYS_ISING) return fail(c, SADMC_E_ARG, "Ising walkers have spins, not coordinates");
   const int n = b->p.n;
+  std::vector<double> p((size_t)3 * b->npad);
+  HIPCHECK(c, fetch(c, p.data(), b->d_pos + (int64_t)w * 3 * b->npad, sizeof(double) * p.size()));
   for (int d = 0; d < 3; d++)
-    HIPCHECK(c, hipMemcpyAsync(coords + (size_t)d * n, b->d_pos + ((int64_t)w * 3 + d) * b->npad, sizeof(double) * n,
-                               hipMemcpyDeviceToHost, c->stream));
-  HIPCHECK(c, hipStreamSynchronize(c->stream));
+    for (int j = 0; j < n; j++) coords[d * n + j] = p[(size_t)d * b->npad + j];
   return SADMC_OK;
 }
 
@@ -1992,8 +2011,7 @@ int sadmc_bin_spins(sadmc_ctx *c, int32_t set, int32_t w, int8_t *spins) {
   if (!b || !spins || w < 0 || w >= b->W) return fail(c, SADMC_E_ARG, "no such binning walker or null output");
   if (b->sys != SYS_ISING) return fail(c, SADMC_E_ARG, "only Ising walkers have spins");
   uint64_t bits = 0;
-  HIPCHECK(c, hipMemcpyAsync(&bits, b->d_spins + w, sizeof bits, hipMemcpyDeviceToHost, c->stream));
-  HIPCHECK(c, hipStreamSynchronize(c->stream));
+  HIPCHECK(c, fetch(c, &bits, b->d_spins + w, sizeof bits));
   const int n = b->p.n;
   for (int k = 0; k < n * n; k++) spins[k] = ((bits >> k) & 1ULL) ? 1 : -1;
   return SADMC_OK;
@@ -2329,8 +2347,7 @@ int sadmc_zmc_replicas(sadmc_ctx *c, int32_t id, int32_t s, int32_t max_out, sad
   ZmcHost *z = zmc_get(c, id);
   if (!z || s < 0 || s >= z->S) return fail(c, SADMC_E_ARG, "no such replica run");
   ZSim sim;
-  HIPCHECK(c, hipMemcpyAsync(&sim, z->d_sim + s, sizeof sim, hipMemcpyDeviceToHost, c->stream));
-  HIPCHECK(c, hipStreamSynchronize(c->stream));
+  HIPCHECK(c, fetch(c, &sim, z->d_sim + s, sizeof sim));
   if (count) *count = sim.R;
   if (out) {
     const int k = std::min(max_out, sim.R);
@@ -2374,8 +2391,7 @@ int sadmc_zmc_spins(sadmc_ctx *c, int32_t id, int32_t s, int32_t r, int8_t *spin
   int rc = zmc_slot(c, z, s, r, &w);
   if (rc) return rc;
   uint64_t b = 0;
-  HIPCHECK(c, hipMemcpyAsync(&b, z->d_spins + w, sizeof b, hipMemcpyDeviceToHost, c->stream));
-  HIPCHECK(c, hipStreamSynchronize(c->stream));
+  HIPCHECK(c, fetch(c, &b, z->d_spins + w, sizeof b));
   for (int k = 0; k < z->n * z->n; k++) spins[k] = ((b >> k) & 1ULL) ? 1 : -1;
   return SADMC_OK;
 }
@@ -2385,8 +2401,7 @@ int sadmc_zmc_state(sadmc_ctx *c, int32_t id, int32_t s, uint64_t *rng, uint64_t
   ZmcHost *z = zmc_get(c, id);
   if (!z || s < 0 || s >= z->S) return fail(c, SADMC_E_ARG, "no such replica run");
   ZSim sim;
-  HIPCHECK(c, hipMemcpyAsync(&sim, z->d_sim + s, sizeof sim, hipMemcpyDeviceToHost, c->stream));
-  HIPCHECK(c, hipStreamSynchronize(c->stream));
+  HIPCHECK(c, fetch(c, &sim, z->d_sim + s, sizeof sim));
   if (rng) {
     rng[0] = sim.rng[0];
     rng[1] = sim.rng[1];
