@@ -197,7 +197,7 @@ struct Engine {
   int32_t pw;
   double ptx, pty, ptz, pe, pdabse;
   // learned move: weights and this walker's exchange row in LDS, ln H
-  const uint16_t *PW;
+  const float *PW;
   float *XC;
   double lnh;
   // this move's SAD gamma (computed again if the move changes lambda or N_s),
@@ -763,17 +763,25 @@ struct Engine {
   }
 
   // Features of the group's atoms around (px, py, pz), skipping atom w;
-  // positions are read from the LDS mirror to keep registers free.
+  // positions are read from the LDS mirror to keep registers free.  The slots
+  // run side by side, as the pair loops' do; a slot without an atom adds +0 to
+  // sums that are never negative.
   SADMC_DF void features(double px, double py, double pz, int w, float *f) {
 #pragma unroll
     for (int c = 0; c < kPropNF; c++) f[c] = 0.0f;
-#pragma unroll 1
-    for (int k = 0; k < K; k++) {
-      int j = lane + G * k;
-      if (j < n && j != w) {
-        float a = (float)(lx[j] - px), b = (float)(ly[j] - py), c = (float)(lz[j] - pz);
-        feature_add(a * a + b * b + c * c, f);
-      }
+    auto slot = [&](int k) {
+      const int j = lane + G * k;
+      const bool use = (j < n) & (j != w);
+      const int jr = 2 * k > KMAX && j >= n ? 0 : j;  // as in lj_lane_sum
+      const float a = (float)(lx[jr] - px), b = (float)(ly[jr] - py), c = (float)(lz[jr] - pz);
+      const float r = __builtin_amdgcn_sqrtf(a * a + b * b + c * c);
+      feature_add(use ? r : kPropFar, f);
+    };
+#pragma unroll
+    for (int k = 0; k < kFirst; k++) slot(k);
+    if (kFirst < KMAX && K > kFirst) {
+#pragma unroll
+      for (int k = kFirst; k < KMAX; k++) slot(k);
     }
 #pragma unroll
     for (int c = 0; c < kPropNF; c++) f[c] = group_sum_f32(f[c], G);

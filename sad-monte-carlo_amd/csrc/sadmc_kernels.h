@@ -326,9 +326,9 @@ static hipError_t launch_km(int meth, int kmax, KernelKind kk, const SetArgs &a,
 }
 
 // ---------------------------------------------------------- learned move
-// LDS: the positions of the 64/G walkers, then the network weights as BF16
-// (in the first half of a region of kPropLds floats), then 32 floats per
-// walker for the hidden-layer exchange of the non-matrix-core form.
+// LDS: the positions of the 64/G walkers, then the network weights as float
+// (kPropLdsF of them), then 32 floats per walker for the hidden-layer exchange
+// of the non-matrix-core form.
 // Two waves per SIMD: the register budget the 16384-walker sets need.  GC
 // as in k_run (the SAD kernels of 2 to 8 atoms per lane at 4, 8 or 16 lanes
 // have it fixed at compile time: fewer scalar spills, +10 % for LJ38 at 8).
@@ -338,14 +338,14 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 2))) void
   extern __shared__ double lds[];
   const int G = GC ? GC : a.G, per = 64 / G;
   float *lw = (float *)(lds + per * 3 * a.npad);
-  load_weights_bf16(a.mlp, (uint16_t *)lw);
+  load_weights_rows(a.mlp, lw);
   const int group = threadIdx.x / G;
   const int lane = threadIdx.x & (G - 1);
   const int walker = blockIdx.x * per + group;
   if (walker >= a.W) return;
   Engine<SYS_LJ, KMAX, PREC, METH, 1, GC> e;
-  e.PW = (const uint16_t *)lw;
-  e.XC = lw + kPropLds + group * kPropH;
+  e.PW = lw;
+  e.XC = lw + kPropLdsF + group * kPropH;
   e.load(a, walker, lane, lds + group * 3 * a.npad);
   e.run(moves);
   e.store(walker);
@@ -355,11 +355,11 @@ template <int KMAX, int PREC, int METH>
 __global__ __launch_bounds__(64) void k_plan_learned(SetArgs a, int walker, Pending *out) {
   extern __shared__ double lds[];
   float *lw = (float *)(lds + 3 * a.npad);
-  load_weights_bf16(a.mlp, (uint16_t *)lw);
+  load_weights_rows(a.mlp, lw);
   if ((int)threadIdx.x >= a.G) return;
   Engine<SYS_LJ, KMAX, PREC, METH, 1> e;
-  e.PW = (const uint16_t *)lw;
-  e.XC = lw + kPropLds;
+  e.PW = lw;
+  e.XC = lw + kPropLdsF;
   e.load(a, walker, threadIdx.x, lds);
   double e2 = 0.0;
   bool some = e.plan_move(0.0, 0.0, e2);
@@ -395,9 +395,9 @@ template <int KMAX, int PREC, int METH>
 static hipError_t launch_learned_t(KernelKind kk, const SetArgs &a, const LaunchArgs &la, hipStream_t s) {
   const int G = a.G;
   const int per_block = 64 / G;
-  const size_t wbytes = sizeof(float) * (kPropLds + (size_t)per_block * kPropH);
+  const size_t wbytes = sizeof(float) * (kPropLdsF + (size_t)per_block * kPropH);
   const size_t lds = (size_t)per_block * 3 * a.npad * sizeof(double) + wbytes;
-  const size_t lds1 = (size_t)3 * a.npad * sizeof(double) + sizeof(float) * (kPropLds + kPropH);
+  const size_t lds1 = (size_t)3 * a.npad * sizeof(double) + sizeof(float) * (kPropLdsF + kPropH);
   const dim3 grid((a.W + per_block - 1) / per_block), block(64);
   switch (kk) {
     case KK_RUN:

@@ -22,7 +22,13 @@
 namespace sadmc {
 
 constexpr int kPropNF = 8, kPropH = 32, kPropNP = 1377, kPropNS = 16, kPropR = 2, kPropRec = 24;
-constexpr int kPropLds = 1384;  // floats reserved for the weights in LDS
+constexpr int kPropLds = 1384;  // the weight arrays' padded length
+// The weights in LDS, widened to float once per launch (the network reads
+// them twice a move): in the parameter order, but with the 32 x 32 layer's rows
+// 36 floats apart, so that the 16 rows a matrix step reads as 16-byte pieces
+// fall into different banks.  45 two-byte reads and shifts per evaluation
+// became 15 reads.
+constexpr int kPropRow = 36, kPropLdsF = 1384 + 32 * (kPropRow - 32);
 constexpr float kPropC0 = 0.9f, kPropDC = 1.6f / 7.0f, kPropA = 12.5f;
 constexpr float kPropSMin = -4.605170186f, kPropSMax = 0.0f;
 // parameter offsets
@@ -52,11 +58,13 @@ __device__ __forceinline__ float group_sum_f32(float v, int G) {
   return v;
 }
 
-// Contribution of one neighbour at float distance^2 r2 to the 8 features
+// Contribution of one neighbour at float distance r to the 8 features
 // (hardware square root and exponential: the proposal only has to be the
-// same function at both ends of a move, not correctly rounded).
-__device__ __forceinline__ void feature_add(float r2, float *f) {
-  const float r = __builtin_amdgcn_sqrtf(r2);
+// same function at both ends of a move, not correctly rounded).  At
+// kPropFar every term is exp2 of less than -1e37, which is +0: what a slot
+// without a neighbour adds.
+constexpr float kPropFar = 1e18f;
+__device__ __forceinline__ void feature_add(float r, float *f) {
 #pragma unroll
   for (int k = 0; k < kPropNF; k++) {
     const float d = r - (kPropC0 + (float)k * kPropDC);
@@ -84,69 +92,62 @@ SADMC_DF double prop_lnh(float s, float s_new, float xi2) {
   return 3.0 * ds + 0.5 * (double)xi2 * (1.0 - exp(2.0 * ds));
 }
 
-// Load the BF16 weights into LDS as float (all 64 lanes of the workgroup).
+// Load the BF16 weights into LDS as float, in the parameter order (all 64
+// lanes of the workgroup; kPropNP floats).
 __device__ __forceinline__ void load_weights(const uint16_t *w, float *lw) {
   for (int i = threadIdx.x; i < kPropNP; i += 64) lw[i] = bf16_to_f32(w[i]);
   __syncthreads();
 }
 
-// Copy the BF16 weights into LDS as they are (kPropLds halfwords, the
-// device array's padded length, as 32-bit words; all lanes of a 64-lane
-// workgroup).
-__device__ __forceinline__ void load_weights_bf16(const uint16_t *w, uint16_t *lw) {
-  const uint32_t *src = (const uint32_t *)w;
-  uint32_t *dst = (uint32_t *)lw;
-  for (int i = threadIdx.x; i < kPropLds / 2; i += 64) dst[i] = src[i];
+// The same in the padded layout above (kPropLdsF floats).
+constexpr int kLW2 = 288, kLB2 = kLW2 + 32 * kPropRow, kLW3 = kLB2 + 32, kLB3 = kLW3 + 32;
+__device__ __forceinline__ void load_weights_rows(const uint16_t *w, float *lw) {
+  for (int i = threadIdx.x; i < kPropNP; i += 64) {
+    const int k = i - kW2;
+    const int at = k < 0 ? i : k < 1024 ? kLW2 + k / 32 * kPropRow + k % 32 : kLB2 + (i - kB2);
+    lw[at] = bf16_to_f32(w[i]);
+  }
   __syncthreads();
 }
 
-// The two BF16 values of a 32-bit word as float: the one at the lower
-// address (low half) and the other.
-__device__ __forceinline__ float bf16_lo(uint32_t v) { return __builtin_bit_cast(float, v << 16); }
-__device__ __forceinline__ float bf16_hi(uint32_t v) { return __builtin_bit_cast(float, v & 0xFFFF0000u); }
-
 // Forward pass for one walker whose G lanes all hold the features f; lane l
 // computes hidden units l, l+G, ... and the group exchanges the first layer
-// through `xc` (32 floats of LDS per walker).  W: the BF16 weights in LDS,
-// widened to float in registers (exact), FP32 arithmetic.
-__device__ __forceinline__ float mlp_forward_bf16(const uint16_t *W, float *xc, const float *f, int lane, int G) {
+// through `xc` (32 floats of LDS per walker).  W: the weights in LDS
+// (load_weights_rows), FP32 arithmetic.
+__device__ __forceinline__ float mlp_forward(const float *W, float *xc, const float *f, int lane, int G) {
   for (int u = lane; u < kPropH; u += G) {
-    const uint4 a = *(const uint4 *)(W + kW1 + u * kPropNF);
-    float z = bf16_to_f32(W[kB1 + u]);
-    z += bf16_lo(a.x) * f[0];
-    z += bf16_hi(a.x) * f[1];
-    z += bf16_lo(a.y) * f[2];
-    z += bf16_hi(a.y) * f[3];
-    z += bf16_lo(a.z) * f[4];
-    z += bf16_hi(a.z) * f[5];
-    z += bf16_lo(a.w) * f[6];
-    z += bf16_hi(a.w) * f[7];
+    const float4 *a = (const float4 *)(W + kW1 + u * kPropNF);
+    const float4 a0 = a[0], a1 = a[1];
+    float z = W[kB1 + u];
+    z += a0.x * f[0];
+    z += a0.y * f[1];
+    z += a0.z * f[2];
+    z += a0.w * f[3];
+    z += a1.x * f[4];
+    z += a1.y * f[5];
+    z += a1.z * f[6];
+    z += a1.w * f[7];
     xc[u] = z > 0.0f ? z : 0.0f;
   }
   __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
   const float4 *x4 = (const float4 *)xc;
   float part = 0.0f;
   for (int u = lane; u < kPropH; u += G) {
-    const uint4 *w2 = (const uint4 *)(W + kW2 + u * kPropH);
-    float z = bf16_to_f32(W[kB2 + u]);
+    const float4 *w2 = (const float4 *)(W + kLW2 + u * kPropRow);
+    float z = W[kLB2 + u];
 #pragma unroll
-    for (int k = 0; k < kPropH / 8; k++) {
-      const uint4 w = w2[k];
-      const float4 h0 = x4[2 * k], h1 = x4[2 * k + 1];
-      z += bf16_lo(w.x) * h0.x;
-      z += bf16_hi(w.x) * h0.y;
-      z += bf16_lo(w.y) * h0.z;
-      z += bf16_hi(w.y) * h0.w;
-      z += bf16_lo(w.z) * h1.x;
-      z += bf16_hi(w.z) * h1.y;
-      z += bf16_lo(w.w) * h1.z;
-      z += bf16_hi(w.w) * h1.w;
+    for (int k = 0; k < kPropH / 4; k++) {
+      const float4 w = w2[k], h = x4[k];
+      z += w.x * h.x;
+      z += w.y * h.y;
+      z += w.z * h.z;
+      z += w.w * h.w;
     }
     const float h = z > 0.0f ? z : 0.0f;
-    part += bf16_to_f32(W[kW3 + u]) * h;
+    part += W[kLW3 + u] * h;
   }
   __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-  float s = bf16_to_f32(W[kB3]) + group_sum_f32(part, G);
+  float s = W[kLB3] + group_sum_f32(part, G);
   return s < kPropSMin ? kPropSMin : (s > kPropSMax ? kPropSMax : s);
 }
 
@@ -158,12 +159,12 @@ __device__ __forceinline__ float mlp_forward_bf16(const uint16_t *W, float *xc, 
 // steps of 4 features), layer 2 H2 = W2 H1 (the hidden layer stays where
 // layer 1 left it: step (m, e) takes unit 16m + 4q + e from element e of
 // lane j + 16q), then s = b3 + w3 . relu(H2 + b2) summed over the four lanes
-// of a column.  FP32 products and sums as in mlp_forward_bf16, in another
+// of a column.  FP32 products and sums as in mlp_forward, in another
 // order.
-// W: the BF16 weights in LDS; f: the walker's features in every lane of its
+// W: the weights in LDS (load_weights_rows); f: the walker's features in every lane of its
 // group; l: the lane in the wave.
 typedef float f32x4 __attribute__((ext_vector_type(4)));
-__device__ __forceinline__ float mlp_wave(const uint16_t *W, const float *f, int l, int G) {
+__device__ __forceinline__ float mlp_wave(const float *W, const float *f, int l, int G) {
   const int i = l & 15, q = l >> 4, j = l & 15;  // A row / B and D column, step
   const int g = l & (G - 1);
   const bool col = j < 64 / G;  // column j is a walker of this wave (else its source lane is wrapped and unused)
@@ -177,53 +178,54 @@ __device__ __forceinline__ float mlp_wave(const uint16_t *W, const float *f, int
     const float mine = G >= 8 ? f[g & 7] : f[(4 * st + g) & 7];
     const float got = __shfl(mine, (G * j + ((4 * st + q) & (G - 1))) & 63, 64);
     const float b = col ? got : 0.0f;
-    const float a0 = bf16_to_f32(W[kW1 + i * kPropNF + 4 * st + q]);
-    const float a1 = bf16_to_f32(W[kW1 + (16 + i) * kPropNF + 4 * st + q]);
+    const float a0 = W[kW1 + i * kPropNF + 4 * st + q];
+    const float a1 = W[kW1 + (16 + i) * kPropNF + 4 * st + q];
     acc0 = __builtin_amdgcn_mfma_f32_16x16x4f32(a0, b, acc0, 0, 0, 0);
     acc1 = __builtin_amdgcn_mfma_f32_16x16x4f32(a1, b, acc1, 0, 0, 0);
   }
   float h1[2][4];
+  const f32x4 b10 = *(const f32x4 *)(W + kB1 + 4 * q), b11 = *(const f32x4 *)(W + kB1 + 16 + 4 * q);
 #pragma unroll
   for (int e = 0; e < 4; e++) {
-    const float z0 = acc0[e] + bf16_to_f32(W[kB1 + 4 * q + e]);
-    const float z1 = acc1[e] + bf16_to_f32(W[kB1 + 16 + 4 * q + e]);
+    const float z0 = acc0[e] + b10[e];
+    const float z1 = acc1[e] + b11[e];
     h1[0][e] = z0 > 0.0f ? z0 : 0.0f;
     h1[1][e] = z1 > 0.0f ? z1 : 0.0f;
   }
   f32x4 d0 = zero, d1 = zero;
 #pragma unroll
   for (int m = 0; m < 2; m++) {
+    const f32x4 a0 = *(const f32x4 *)(W + kLW2 + i * kPropRow + 16 * m + 4 * q);
+    const f32x4 a1 = *(const f32x4 *)(W + kLW2 + (16 + i) * kPropRow + 16 * m + 4 * q);
 #pragma unroll
     for (int e = 0; e < 4; e++) {
-      const float a0 = bf16_to_f32(W[kW2 + i * kPropH + 16 * m + 4 * q + e]);
-      const float a1 = bf16_to_f32(W[kW2 + (16 + i) * kPropH + 16 * m + 4 * q + e]);
-      d0 = __builtin_amdgcn_mfma_f32_16x16x4f32(a0, h1[m][e], d0, 0, 0, 0);
-      d1 = __builtin_amdgcn_mfma_f32_16x16x4f32(a1, h1[m][e], d1, 0, 0, 0);
+      d0 = __builtin_amdgcn_mfma_f32_16x16x4f32(a0[e], h1[m][e], d0, 0, 0, 0);
+      d1 = __builtin_amdgcn_mfma_f32_16x16x4f32(a1[e], h1[m][e], d1, 0, 0, 0);
     }
   }
   float part = 0.0f;
 #pragma unroll
   for (int mo = 0; mo < 2; mo++) {
+    const f32x4 b2 = *(const f32x4 *)(W + kLB2 + 16 * mo + 4 * q), w3 = *(const f32x4 *)(W + kLW3 + 16 * mo + 4 * q);
 #pragma unroll
     for (int e = 0; e < 4; e++) {
-      const int u = 16 * mo + 4 * q + e;
-      const float z = (mo == 0 ? d0[e] : d1[e]) + bf16_to_f32(W[kB2 + u]);
-      part += bf16_to_f32(W[kW3 + u]) * (z > 0.0f ? z : 0.0f);
+      const float z = (mo == 0 ? d0[e] : d1[e]) + b2[e];
+      part += w3[e] * (z > 0.0f ? z : 0.0f);
     }
   }
   part += __shfl_xor(part, 16, 64);
   part += __shfl_xor(part, 32, 64);
-  float s = bf16_to_f32(W[kB3]) + part;
+  float s = W[kLB3] + part;
   s = s < kPropSMin ? kPropSMin : (s > kPropSMax ? kPropSMax : s);
   // walker l / G reads its column
   return __shfl(s, l / G, 64);
 }
 
 // The network for the walker of this lane's group: on the matrix cores when
-// every lane of the wave is here and G >= 4, else mlp_forward_bf16.
-__device__ __forceinline__ float mlp_eval(const uint16_t *W, float *xc, const float *f, int lane, int G) {
+// every lane of the wave is here and G >= 4, else mlp_forward.
+__device__ __forceinline__ float mlp_eval(const float *W, float *xc, const float *f, int lane, int G) {
   if (G >= 4 && __builtin_amdgcn_read_exec() == ~0ull) return mlp_wave(W, f, (int)(threadIdx.x & 63), G);
-  return mlp_forward_bf16(W, xc, f, lane, G);
+  return mlp_forward(W, xc, f, lane, G);
 }
 
 }  // namespace sadmc
