@@ -6,12 +6,12 @@
 //   temperature of the replica that owns it (Replica::run_once,
 //   tempering.rs:96-112), with that replica's generator and counters, all
 //   groups at once;
-// - lane 0 of the workgroup then draws the ladder generator's bool and walks
-//   the odd or even neighbour pairs (tempering.rs:288-318) in order, deciding
-//   each swap with the second replica's generator and collecting both
-//   replicas' energies.  A swap exchanges the owners of two slots, so no
-//   positions move; the replica records, the owner tables and the slot
-//   energies live in LDS for the whole launch.
+// - every lane draws the ladder generator's bool, and one lane per odd or
+//   even neighbour pair (tempering.rs:288-318; the pairs share nothing, so
+//   their order does not show) decides its swap with the second replica's
+//   generator and collects both replicas' energies.  A swap exchanges the
+//   owners of two slots, so no positions move; the replica records, the owner
+//   tables and the slot energies live in LDS for the whole launch.
 #define SADMC_KERNEL_TU
 #include "sadmc_kernels.h"
 
@@ -104,11 +104,7 @@ __global__ __launch_bounds__(512) void k_pt(SetArgs a, PtArgs p, uint64_t rounds
     return;
   }
 
-  uint64_t l0 = 0, l1 = 0;
-  if (tid == 0) {
-    l0 = p.lrng[2 * ladder];
-    l1 = p.lrng[2 * ladder + 1];
-  }
+  uint64_t l0 = p.lrng[2 * ladder], l1 = p.lrng[2 * ladder + 1];
   for (uint64_t k = 0; k < rounds; k++) {
     if (active) {
       const int r = rep_of[slot];
@@ -140,37 +136,39 @@ __global__ __launch_bounds__(512) void k_pt(SetArgs a, PtArgs p, uint64_t rounds
       }
     }
     __syncthreads();
-    if (tid == 0) {
-      // rand 0.7's bool is the top bit of next_u32, which rand_xoshiro takes
-      // from the high half of next_u64
-      const int first = (rng_next(l0, l1) >> 63) ? 0 : 1;
-      for (int i = first; i + 1 < R; i += 2) {
-        PtMeta &m0 = meta[i], &m1 = meta[i + 1];
-        const int a0 = slot_of[i], a1 = slot_of[i + 1];
-        const double E0 = se[2 * a0], E1 = se[2 * a1];
-        const double de_db = (E0 - E1) * (1.0 / m0.T - 1.0 / m1.T);
-        bool swap = de_db >= 0.0;
-        if (!swap) {
-          uint64_t u0 = m1.rng0, u1 = m1.rng1;
-          swap = gen_f64(u0, u1) < exp(de_db);
-          m1.rng0 = u0;
-          m1.rng1 = u1;
-        }
-        if (swap) {
-          m0.as += 1;
-          m1.as += 1;
-          slot_of[i] = a1;
-          slot_of[i + 1] = a0;
-          rep_of[a1] = i;
-          rep_of[a0] = i + 1;
-          pt_collect(m0, E1);
-          pt_collect(m1, E0);
-        } else {
-          m0.rs += 1;
-          m1.rs += 1;
-          pt_collect(m0, E0);
-          pt_collect(m1, E1);
-        }
+    // rand 0.7's bool is the top bit of next_u32, which rand_xoshiro takes
+    // from the high half of next_u64 (every lane draws it)
+    const int first = (rng_next(l0, l1) >> 63) ? 0 : 1;
+    // the round's pairs share no replica and no slot, and each is decided with
+    // its second replica's generator: one lane per pair (one lane for all of
+    // them took 160 cycles of a move of 3900)
+    const int i = first + 2 * tid;
+    if (i + 1 < R) {
+      PtMeta &m0 = meta[i], &m1 = meta[i + 1];
+      const int a0 = slot_of[i], a1 = slot_of[i + 1];
+      const double E0 = se[2 * a0], E1 = se[2 * a1];
+      const double de_db = (E0 - E1) * (1.0 / m0.T - 1.0 / m1.T);
+      bool swap = de_db >= 0.0;
+      if (!swap) {
+        uint64_t u0 = m1.rng0, u1 = m1.rng1;
+        swap = gen_f64(u0, u1) < exp(de_db);
+        m1.rng0 = u0;
+        m1.rng1 = u1;
+      }
+      if (swap) {
+        m0.as += 1;
+        m1.as += 1;
+        slot_of[i] = a1;
+        slot_of[i + 1] = a0;
+        rep_of[a1] = i;
+        rep_of[a0] = i + 1;
+        pt_collect(m0, E1);
+        pt_collect(m1, E0);
+      } else {
+        m0.rs += 1;
+        m1.rs += 1;
+        pt_collect(m0, E0);
+        pt_collect(m1, E1);
       }
     }
     __syncthreads();

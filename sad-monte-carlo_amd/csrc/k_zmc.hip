@@ -175,15 +175,6 @@ __global__ __launch_bounds__(64) void k_zmc(ZArgs z, SetArgs a, uint64_t rounds)
       e.err = sErr[slot];
       if (SYS == SYS_ISING) {
         e.spins = spn[slot];
-      } else if (!e.kLdsPos) {
-#pragma unroll
-        for (int k = 0; k < KMAX; k++)
-          if (k < e.K) {
-            const int j = lane + G * k;
-            e.x[k] = e.lx[j];
-            e.y[k] = e.ly[j];
-            e.z[k] = e.lz[j];
-          }
       }
       const int r = rep_of[slot];
       ZMeta m = meta[r];
@@ -269,16 +260,6 @@ __global__ __launch_bounds__(64) void k_zmc(ZArgs z, SetArgs a, uint64_t rounds)
             }
           }
           __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-          if (!e.kLdsPos) {
-#pragma unroll
-            for (int k = 0; k < KMAX; k++)
-              if (k < e.K) {
-                const int j = lane + G * k;
-                e.x[k] = e.lx[j];
-                e.y[k] = e.ly[j];
-                e.z[k] = e.lz[j];
-              }
-          }
         }
         e.E = e.full_energy();
         low = m.max_e;

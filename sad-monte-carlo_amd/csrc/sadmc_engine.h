@@ -5,8 +5,8 @@
 // Layout.  Every lane of a group holds the walker's hot scalar state in
 // registers (identical values: all lanes execute the same bookkeeping, so no
 // broadcast is ever needed).  For LJ/WCA, lane l of the group owns atoms l,
-// l+G, l+2G, ... (K slots, SoA registers); the group also keeps an LDS mirror
-// of all N positions so any lane can read the moved atom.  The energy
+// l+G, l+2G, ... (K slots); the positions of all N atoms are an SoA tile in LDS,
+// so any lane can read the moved atom.  The energy
 // difference of a move is a per-lane partial sum over the lane's atoms
 // followed by an xor butterfly across the G lanes.  Ising uses one lane per
 // walker (G = 1) with the N*N <= 64 spins bit-packed in one 64-bit register.
@@ -139,18 +139,13 @@ struct Engine {
   int wk;  // the walker's index in its set
   // system
   double *lx, *ly, *lz;
-  // This lane's atoms in registers, or (kLdsPos) read from the LDS mirror:
-  // the learned move, WCA and groups with many atoms per lane keep their
-  // registers for the rest of the state.
-  static constexpr bool kLdsPos = MV == 1 || SYS == SYS_WCA || KMAX >= 8;
-  double x[KMAX], y[KMAX], z[KMAX];
+  // The positions stay in LDS (one tile per walker): copies of a lane's atoms
+  // in registers cost 24 of them and 30 selects per accepted move, more than
+  // the reads (1 to 4 % of the walker kernels).
   // The slots a pair loop runs without asking for K, so that their chains
   // interleave: K > KMAX/2 always, and up to 4 slots the one too many is
   // cheaper than a branch.
   static constexpr int kFirst = KMAX <= 4 ? KMAX : KMAX / 2 + 1;
-  SADMC_DF double xk(int k) const { return kLdsPos ? lx[lane + G * k] : x[k]; }
-  SADMC_DF double yk(int k) const { return kLdsPos ? ly[lane + G * k] : y[k]; }
-  SADMC_DF double zk(int k) const { return kLdsPos ? lz[lane + G * k] : z[k]; }
   uint64_t spins;
   double R2, L, halfL;
   // EnergyMC scalars
@@ -236,22 +231,11 @@ struct Engine {
       const double *P = a.pos + (int64_t)walker * 3 * a.npad;
 #pragma unroll
       for (int k = 0; k < KMAX; k++) {
-        if (!kLdsPos) {
-          x[k] = 0.0;
-          y[k] = 0.0;
-          z[k] = 0.0;
-        }
         if (k < K) {
           int j = lane + G * k;
-          const double vx = P[j], vy = P[a.npad + j], vz = P[2 * a.npad + j];
-          if (!kLdsPos) {
-            x[k] = vx;
-            y[k] = vy;
-            z[k] = vz;
-          }
-          lx[j] = vx;
-          ly[j] = vy;
-          lz[j] = vz;
+          lx[j] = P[j];
+          ly[j] = P[a.npad + j];
+          lz[j] = P[2 * a.npad + j];
         }
       }
       __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
@@ -373,9 +357,9 @@ struct Engine {
       for (int k = 0; k < KMAX; k++) {
         if (k < K) {
           int j = lane + G * k;
-          P[j] = xk(k);
-          P[args().npad + j] = yk(k);
-          P[2 * args().npad + j] = zk(k);
+          P[j] = lx[j];
+          P[args().npad + j] = ly[j];
+          P[2 * args().npad + j] = lz[j];
         }
       }
     }
@@ -541,7 +525,7 @@ struct Engine {
         }
       return e;
     }
-    // rare: one small loop from the LDS mirror instead of KMAX unrolled ones
+    // rare: one small loop instead of KMAX unrolled ones
     double acc = 0.0;
 #pragma unroll 1
     for (int i = lane; i < n; i += G) {
@@ -762,10 +746,9 @@ struct Engine {
     return some;
   }
 
-  // Features of the group's atoms around (px, py, pz), skipping atom w;
-  // positions are read from the LDS mirror to keep registers free.  The slots
-  // run side by side, as the pair loops' do; a slot without an atom adds +0 to
-  // sums that are never negative.
+  // Features of the group's atoms around (px, py, pz), skipping atom w.  The
+  // slots run side by side, as the pair loops' do; a slot without an atom adds
+  // +0 to sums that are never negative.
   SADMC_DF void features(double px, double py, double pz, int w, float *f) {
 #pragma unroll
     for (int c = 0; c < kPropNF; c++) f[c] = 0.0f;
@@ -801,7 +784,7 @@ struct Engine {
       const bool use = (j < n) & (j != w);
       // slots that K may not reach read atom 0 (and are dropped)
       const int jr = 2 * k > KMAX && j >= n ? 0 : j;
-      const double xj = kLdsPos ? lx[jr] : x[k], yj = kLdsPos ? ly[jr] : y[k], zj = kLdsPos ? lz[jr] : z[k];
+      const double xj = lx[jr], yj = ly[jr], zj = lz[jr];
       double t;
       if (PREC == 1) {
         const float an = (float)(xj - tx), bn = (float)(yj - ty), cn = (float)(zj - tz);
@@ -822,8 +805,7 @@ struct Engine {
     }
     return acc;
   }
-  // The same with the divisions; hardly ever needed, so a small loop over the
-  // LDS mirror.
+  // The same with the divisions; hardly ever needed, so a small loop.
   SADMC_DF double lj_lane_sum_div(int w, double tx, double ty, double tz, double fx, double fy, double fz) {
     double acc = 0.0;
 #pragma unroll 1
@@ -1005,17 +987,7 @@ struct Engine {
       spins ^= (1ULL << pw);
       return;
     }
-    int owner = pw & (G - 1);
-    int slot = pw / G;
-#pragma unroll
-    for (int k = 0; k < KMAX; k++) {
-      if (!kLdsPos && lane == owner && k == slot) {
-        x[k] = ptx;
-        y[k] = pty;
-        z[k] = ptz;
-      }
-    }
-    if (lane == owner) {
+    if (lane == 0) {
       lx[pw] = ptx;
       ly[pw] = pty;
       lz[pw] = ptz;
