@@ -12,9 +12,12 @@
 // covering each bin.
 //
 // k_entropy_walker: one wavefront per walker computes i_lo, i_hi, <H> and the
-// window mean.  k_entropy_bins: one lane per global bin loops over the
+// window mean.  k_entropy_bins: two global bins per lane, looping over the
 // walkers; consecutive lanes read consecutive bins of the same walker, so
 // every load of the 16-byte hot records is coalesced.
+// Both are bound by HBM: 16384 LJ31 walkers of 7900 bins are 2.07 GB a pass,
+// 377 us for the first (5.5 TB/s; it read the window a second time before)
+// and about 430 us for the second.
 #include "sadmc_kernels.h"
 
 namespace sadmc {
@@ -59,23 +62,40 @@ __global__ __launch_bounds__(64) void k_entropy_walker(const sadmc_walker_state 
     return best;
   };
   const int64_t ilo = nearest(s.too_lo), ihi = nearest(s.too_hi);
-  // four loads in flight per lane; the additions keep the i order
-  double hsum = 0.0;
-  for (int64_t i0 = ilo + threadIdx.x; i0 <= ihi; i0 += 256) {
-    uint64_t h[4];
+  // Where the window lies inside the walker's range (the default one does),
+  // its values are plain ln w and one sweep serves both sums: lane l takes the
+  // bins g = ga + l (mod 64), as the window's sum below does, and the counts
+  // add up exactly in any order.  Otherwise the window's sweep follows once <H>
+  // is known.  Eight loads in flight per lane.
+  const int64_t a0 = ga - off, b0 = gb - off;
+  const bool inside = a0 >= 0 && b0 <= len && bmin + ((double)a0 + 0.5) * width >= s.too_lo &&
+                      bmin + ((double)(b0 - 1) + 0.5) * width <= s.too_hi;
+  double hsum = 0.0, csum = 0.0;
+  int64_t ccount = 0;
+  const int64_t ifrom = inside && a0 < ilo ? a0 : ilo, ito = inside && b0 - 1 > ihi ? b0 - 1 : ihi;
+  for (int64_t i0 = ifrom + ((a0 + (int64_t)threadIdx.x - ifrom) & 63); i0 <= ito; i0 += 512) {
+    HotBin h[8];
 #pragma unroll
-    for (int u = 0; u < 4; u++) h[u] = i0 + 64 * u <= ihi ? H[i0 + 64 * u].hist : 0;
+    for (int u = 0; u < 8; u++) {
+      h[u].lnw = 0.0;
+      h[u].hist = 0;
+      if (i0 + 64 * u <= ito) h[u] = H[i0 + 64 * u];
+    }
 #pragma unroll
-    for (int u = 0; u < 4; u++)
-      if (i0 + 64 * u <= ihi) hsum += (double)h[u];
+    for (int u = 0; u < 8; u++) {
+      const int64_t i = i0 + 64 * u;
+      if (i >= ilo && i <= ihi) hsum += (double)h[u].hist;
+      if (inside && i >= a0 && i < b0) {
+        csum += h[u].lnw;
+        ccount += 1;
+      }
+    }
   }
   for (int d = 32; d >= 1; d >>= 1) hsum += __shfl_xor(hsum, d, 64);
   const double mean_hist = hsum / (double)(ihi - ilo + 1);
   const double lnw_lo = H[ilo].lnw, lnw_hi = H[ihi].lnw;
   // the window mean of the extended S; every window bin must carry an estimate
-  double csum = 0.0;
-  int64_t ccount = 0;
-  for (int64_t g = ga + threadIdx.x; g < gb; g += 64) {
+  for (int64_t g = ga + threadIdx.x; g < gb && !inside; g += 64) {
     const int64_t i = g - off;
     if (i < 0 || i >= len) continue;
     const HotBin b = H[i];
@@ -114,55 +134,75 @@ __global__ __launch_bounds__(64) void k_entropy_walker(const sadmc_walker_state 
   }
 }
 
-// One lane per grid bin and one block row per chunk of walkers: partial
-// sums over the chunk's walkers, so that the grid fills the device.
+// Each lane takes kBinsPerLane grid bins, 256 apart, and each block row a
+// chunk of walkers: partial sums over the chunk's walkers in their order.  The
+// shape is measured (16384 LJ31 walkers, whole call): bins per lane x walkers
+// in flight 1 x 4 1098 us, 1 x 8 1085, 2 x 4 912, 2 x 8 1090, 3 x 4 969, 4 x 2
+// 1003, 4 x 4 982.
+constexpr int kBinsPerLane = 2, kWalkersInFlight = 4;
 __global__ __launch_bounds__(256) void k_entropy_bins(const EntropyWalker *ew, int W, const HotBin *hot, int64_t cap,
                                                       double width, int64_t ng, int chunks, double *psum,
                                                       int64_t *pcnt) {
-  const int64_t g = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  if (g >= ng) return;
+  const int64_t g0 = (int64_t)blockIdx.x * (256 * kBinsPerLane) + threadIdx.x;
   const int c = blockIdx.y;
   const int w0 = (int)((int64_t)W * c / chunks), w1 = (int)((int64_t)W * (c + 1) / chunks);
-  double sum = 0.0;
-  int64_t n = 0;
-  for (int w4 = w0; w4 < w1; w4 += 4) {
-    // the records of up to four walkers in flight, used in walker order
-    HotBin bq[4];
+  double sum[kBinsPerLane];
+  int32_t n[kBinsPerLane];
 #pragma unroll
-    for (int u = 0; u < 4; u++) {
-      const int w = w4 + u;
-      bq[u].lnw = 0.0;
-      bq[u].hist = 0;
-      if (w < w1) {
-        const int64_t i = g - ew[w].off;
-        if (ew[w].ok && i >= 0 && i < ew[w].len) bq[u] = hot[(int64_t)w * cap + ew[w].base + i];
+  for (int b = 0; b < kBinsPerLane; b++) {
+    sum[b] = 0.0;
+    n[b] = 0;
+  }
+  for (int wq = w0; wq < w1; wq += kWalkersInFlight) {
+    // the records of a few walkers in flight, used in walker order
+    HotBin bq[kWalkersInFlight][kBinsPerLane];
+#pragma unroll
+    for (int u = 0; u < kWalkersInFlight; u++) {
+      const int w = wq + u < w1 ? wq + u : w1 - 1;
+      const int64_t off = ew[w].off, len = ew[w].ok ? ew[w].len : 0;
+      const HotBin *H = hot + (int64_t)w * cap + ew[w].base;
+#pragma unroll
+      for (int b = 0; b < kBinsPerLane; b++) {
+        const int64_t i = g0 + 256 * b - off;
+        bq[u][b].lnw = 0.0;
+        bq[u][b].hist = 0;
+        if (i >= 0 && i < len) bq[u][b] = H[i];
       }
     }
 #pragma unroll
-    for (int u = 0; u < 4; u++) {
-      const int w = w4 + u;
+    for (int u = 0; u < kWalkersInFlight; u++) {
+      const int w = wq + u;
       if (w >= w1) continue;
       const EntropyWalker e = ew[w];
-      const int64_t i = g - e.off;
-      if (!e.ok || i < 0 || i >= e.len) continue;
-      const HotBin b = bq[u];
-      const double E = e.bmin + ((double)i + 0.5) * width;
-      double v;
-      if (E < e.too_lo) {
-        if (b.hist == 0) continue;
-        v = e.lnw_lo + (E - e.too_lo) / e.min_T + log((double)b.hist / e.mean_hist);
-      } else if (E > e.too_hi) {
-        if (b.hist == 0) continue;
-        v = e.lnw_hi + log((double)b.hist / e.mean_hist);
-      } else {
-        v = b.lnw;
+      const int64_t len = e.ok ? e.len : 0;
+#pragma unroll
+      for (int b = 0; b < kBinsPerLane; b++) {
+        const int64_t i = g0 + 256 * b - e.off;
+        const double E = e.bmin + ((double)i + 0.5) * width;
+        double v = bq[u][b].lnw;
+        bool have = i >= 0 && i < len;
+        if (have && (E < e.too_lo || E > e.too_hi)) {
+          have = bq[u][b].hist != 0;
+          if (have) {
+            const double l = log((double)bq[u][b].hist / e.mean_hist);
+            v = E < e.too_lo ? e.lnw_lo + (E - e.too_lo) / e.min_T + l : e.lnw_hi + l;
+          }
+        }
+        if (have) {
+          sum[b] += v - e.c;
+          n[b] += 1;
+        }
       }
-      sum += v - e.c;
-      n += 1;
     }
   }
-  psum[(int64_t)c * ng + g] = sum;
-  pcnt[(int64_t)c * ng + g] = n;
+#pragma unroll
+  for (int b = 0; b < kBinsPerLane; b++) {
+    const int64_t g = g0 + 256 * b;
+    if (g < ng) {
+      psum[(int64_t)c * ng + g] = sum[b];
+      pcnt[(int64_t)c * ng + g] = n[b];
+    }
+  }
 }
 
 // The chunks' partial sums, combined in chunk order.
@@ -307,7 +347,8 @@ hipError_t launch_entropy(const sadmc_walker_state *ws, const HotBin *hot, int W
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
   const unsigned bx = (unsigned)((ng + 255) / 256);
-  hipLaunchKernelGGL(k_entropy_bins, dim3(bx, (unsigned)chunks), dim3(256), 0, s, (const EntropyWalker *)ew, W, hot,
+  const unsigned bins_x = (unsigned)((ng + 256 * kBinsPerLane - 1) / (256 * kBinsPerLane));
+  hipLaunchKernelGGL(k_entropy_bins, dim3(bins_x, (unsigned)chunks), dim3(256), 0, s, (const EntropyWalker *)ew, W, hot,
                      cap, width, ng, chunks, psum, pcnt);
   e = hipGetLastError();
   if (e != hipSuccess) return e;
