@@ -11,7 +11,8 @@
 // followed by an xor butterfly across the G lanes.  Ising uses one lane per
 // walker (G = 1) with the N*N <= 64 spins bit-packed in one 64-bit register.
 //
-// Bins.  A walker's bins are a fixed window of `cap` 64-byte records in HBM.
+// Bins.  A walker's bins are a fixed window of `cap` records in HBM, split by
+// use (HotBin, ColdBin, the arrays beside them).
 // Logical bin i lives in physical slot base + i; the reference's front
 // insertion (energy.rs:400-420) becomes base -= 1, and the slots outside the
 // window are zero from allocation, which is exactly the value the reference

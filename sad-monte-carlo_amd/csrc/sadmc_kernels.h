@@ -1,10 +1,12 @@
 // Kernel templates and per-system launch entry points.
 //
-// Launch shape: one 64-lane wavefront per workgroup; a workgroup holds 64/G
-// walkers of one set, G lanes each (G = 1 for Ising), and the LDS mirror of
-// their positions: (64/G) * 3 * npad doubles.  The run kernel is persistent
-// over the K moves of a batch: walker state is read from HBM once, kept in
-// registers for the whole batch, and written back once.
+// Launch shape: a 64-lane wavefront holds up to 64/G walkers of one set, G
+// lanes each (G = 1 for Ising), and their positions in LDS, 3 * npad doubles a
+// walker (the only copy during a launch).  A workgroup is one wavefront, the
+// run kernel's and the batched kernel's also two or four, and the run kernel
+// gives small sets' waves fewer walkers (walkers_per_wave).  The run kernel is
+// persistent over the K moves of a batch: walker state is read from HBM once,
+// kept in registers and LDS for the whole batch, and written back once.
 #pragma once
 
 #include "sadmc_engine.h"
