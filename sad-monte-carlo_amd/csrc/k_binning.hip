@@ -72,10 +72,10 @@ __device__ __forceinline__ double shfl_f64(double v, int d) {
 
 // LIN: the linear interpolation of binning/linear.rs instead of the
 // histogram of binning/histogram.rs.
-template <int SYS, int KMAX, bool LIN>
+template <int SYS, int KMAX, bool LIN, bool SH>
 struct BinWalker {
   using CT = typename std::conditional<LIN, double, uint64_t>::type;
-  Engine<SYS, KMAX, 0, M_CAN> e;
+  Engine<SYS, KMAX, 0, M_CAN, 0, 0, SH> e;
   const BinArgs *Bp;
   sadmc_bbin *B;  // this walker's window of bins
   BC<CT> *bc;     // [kBinStats] in LDS
@@ -1225,17 +1225,17 @@ struct BinWalker {
 
 // `per` walkers a wave, as for the main engine's run kernel; registers for two
 // waves per SIMD, which 16384 walkers at 8 lanes need.
-template <int SYS, int KMAX, bool LIN>
+template <int SYS, int KMAX, bool LIN, bool SH>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void k_bin(BinArgs ba, SetArgs sa, uint64_t nmoves, int init, int per) {
   extern __shared__ double lds[];
-  const int G = sa.G, group = threadIdx.x / G;
+  const int G = sa.G, group = threadIdx.x / (SH ? G * KMAX : G);
   const int lane = threadIdx.x & (G - 1);
   const int walker = blockIdx.x * per + group;
   const bool held = group < per && walker < sa.W;
   double *tile = lds + (SYS == SYS_ISING ? 0 : group * 3 * sa.npad);
   char *stats = (char *)(lds + (SYS == SYS_ISING ? 0 : per * 3 * sa.npad)) +
                 group * (int)(kBinStats * sizeof(BC<uint64_t>));
-  BinWalker<SYS, KMAX, LIN> b;
+  BinWalker<SYS, KMAX, LIN, SH> b;
   if (held) {
     b.load(ba, sa, walker, lane, tile, stats);
   } else {
@@ -1255,10 +1255,20 @@ static hipError_t launch_bin_t(const BinArgs &ba, const SetArgs &sa, uint64_t mo
   const int blocks = (sa.W + per - 1) / per;
   const size_t lds = (SYS == SYS_ISING ? 0 : sizeof(double) * 3 * (size_t)per * sa.npad) +
                      (size_t)per * kBinStats * sizeof(BC<uint64_t>);
-  if (ba.linear)
-    hipLaunchKernelGGL((k_bin<SYS, KMAX, true>), dim3(blocks), dim3(64), lds, s, ba, sa, moves, init, per);
-  else
-    hipLaunchKernelGGL((k_bin<SYS, KMAX, false>), dim3(blocks), dim3(64), lds, s, ba, sa, moves, init, per);
+  const auto go = [&](auto share) {
+    constexpr bool SH = decltype(share)::value;
+    if (ba.linear)
+      hipLaunchKernelGGL((k_bin<SYS, KMAX, true, SH>), dim3(blocks), dim3(64), lds, s, ba, sa, moves, init, per);
+    else
+      hipLaunchKernelGGL((k_bin<SYS, KMAX, false, SH>), dim3(blocks), dim3(64), lds, s, ba, sa, moves, init, per);
+  };
+  if constexpr (SYS != SYS_ISING && KMAX > 1) {
+    if (lanes_to_share(per, sa.G, KMAX)) {
+      go(std::true_type{});
+      return hipGetLastError();
+    }
+  }
+  go(std::false_type{});
   return hipGetLastError();
 }
 

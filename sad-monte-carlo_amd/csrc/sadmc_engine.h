@@ -129,8 +129,13 @@ __device__ __forceinline__ uint32_t sample_zone(uint64_t &s0, uint64_t &s1, uint
 // MV = 1: the learned Gaussian move with its Hastings term (LJ only).
 // GC > 0: the lanes per walker fixed at compile time (must equal the set's
 // G), which folds the group sums, lane indices and atom-slot arithmetic.
-template <int SYS, int KMAX, int PREC, int METH, int MV = 0, int GC = 0>
+// SH: a wave with few walkers, in which kShare = KMAX lanes stand for each of a
+// group's G, all with the walker's whole state, and share its pair terms, one
+// atom slot a lane.
+template <int SYS, int KMAX, int PREC, int METH, int MV = 0, int GC = 0, bool SH = false>
 struct Engine {
+  static constexpr int kShare = SH ? KMAX : 1;
+  SADMC_DF static int wave_lane() { return (int)(threadIdx.x & 63); }
   const SetArgs *Ap;  // kernel argument segment (uniform; read with scalar loads)
   SADMC_DF const SetArgs &args() const { return *Ap; }
   int lane, G, K, n;
@@ -557,8 +562,8 @@ struct Engine {
   // estimate trips (LJ every 10 N accepted moves, WCA every 10), and a group
   // alone runs through the N^2/2 pairs with 64 - G lanes idle.
   SADMC_DF double wave_full_energy(int leader) const {
-    const int R = 64 / G, c = (int)(threadIdx.x & 63) / G;
-    const double *X = lx + (leader / G - c) * 3 * args().npad, *Y = X + args().npad, *Z = Y + args().npad;
+    const int R = 64 / G, c = wave_lane() / G, GP = G * kShare;
+    const double *X = lx + (leader / GP - wave_lane() / GP) * 3 * args().npad, *Y = X + args().npad, *Z = Y + args().npad;
     const double Lw = SYS == SYS_WCA ? __shfl(L, leader, 64) : 0.0, hw = 0.5 * Lw;
     constexpr int U = 4;  // terms in flight per lane
     double acc = 0.0;
@@ -622,12 +627,12 @@ struct Engine {
     if (!todo) return;
     bool serial = need;
     if (SYS != SYS_ISING && G < 64 && __ballot(1) == ~0ULL) {
-      const int mine = (int)(threadIdx.x & 63) / G;
+      const int GP = G * kShare, mine = wave_lane() / GP;
       while (todo) {
         const int leader = (int)__builtin_ctzll(todo);
-        todo &= ~(((1ULL << G) - 1) << (leader / G * G));
+        todo &= ~((~0ULL >> (64 - GP)) << (leader / GP * GP));
         const double e = wave_full_energy(leader);
-        if (leader / G == mine) {
+        if (leader / GP == mine) {
           E = e;
           serial = SYS == SYS_LJ && e != e;
         }
@@ -714,26 +719,37 @@ struct Engine {
     if (SYS == SYS_LJ) {
       acc = lj_lane_diff(w, tx, ty, tz, fx, fy, fz);
     } else {
-      auto slot = [&](int k) {
-        const int j = lane + G * k;
-        const bool use = (j < n) & (j != w);
-        const int jr = 2 * k > KMAX && j >= n ? 0 : j;  // as in lj_lane_sum
+      double vn, vo;
+      auto terms = [&](int jr) {
         const double xj = lx[jr], yj = ly[jr], zj = lz[jr];
-        const double vn = wca_pair_fast(norm2(min_image(xj - tx, L, halfL), min_image(yj - ty, L, halfL),
-                                              min_image(zj - tz, L, halfL)),
-                                        args().rc2);
-        const double vo = wca_pair_fast(norm2(min_image(xj - fx, L, halfL), min_image(yj - fy, L, halfL),
-                                              min_image(zj - fz, L, halfL)),
-                                        args().rc2);
-        const double na = acc + (vn - vo), nb = accabs + (vn + vo);
-        acc = use ? na : acc;
-        accabs = use ? nb : accabs;
+        vn = wca_pair_fast(norm2(min_image(xj - tx, L, halfL), min_image(yj - ty, L, halfL),
+                                 min_image(zj - tz, L, halfL)),
+                           args().rc2);
+        vo = wca_pair_fast(norm2(min_image(xj - fx, L, halfL), min_image(yj - fy, L, halfL),
+                                 min_image(zj - fz, L, halfL)),
+                           args().rc2);
       };
+      if constexpr (SH) {
+        const int j = lane + G * (wave_lane() / G & (KMAX - 1));
+        const bool use = (j < n) & (j != w);
+        terms(use ? j : 0);
+        acc = shared_sum(use ? vn - vo : 0.0);
+        accabs = shared_sum(use ? vn + vo : 0.0);
+      } else {
+        auto slot = [&](int k) {
+          const int j = lane + G * k;
+          const bool use = (j < n) & (j != w);
+          terms(2 * k > KMAX && j >= n ? 0 : j);  // as in lj_lane_sum
+          const double na = acc + (vn - vo), nb = accabs + (vn + vo);
+          acc = use ? na : acc;
+          accabs = use ? nb : accabs;
+        };
 #pragma unroll
-      for (int k = 0; k < kFirst; k++) slot(k);
-      if (kFirst < KMAX && K > kFirst) {
+        for (int k = 0; k < kFirst; k++) slot(k);
+        if (kFirst < KMAX && K > kFirst) {
 #pragma unroll
-        for (int k = kFirst; k < KMAX; k++) slot(k);
+          for (int k = kFirst; k < KMAX; k++) slot(k);
+        }
       }
     }
     double e = E + group_sum(acc, G);
@@ -771,6 +787,19 @@ struct Engine {
     for (int c = 0; c < kPropNF; c++) f[c] = group_sum_f32(f[c], G);
   }
 
+  // The sum over a lane's slots of the terms its KMAX lanes hold, in slot
+  // order.  A slot without a term holds +0, which changes no sum here (none
+  // is -0).
+  SADMC_DF double shared_sum(double t) const {
+    const int src = (wave_lane() & ~(G * KMAX - 1)) + lane;
+    double v[KMAX], acc = 0.0;
+#pragma unroll
+    for (int k = 0; k < KMAX; k++) v[k] = __shfl(t, src + k * G, 64);
+#pragma unroll
+    for (int k = 0; k < KMAX; k++) acc += v[k];
+    return acc;
+  }
+
   // This lane's sum of the pair-term differences V(|x_j - t|^2) -
   // V(|x_j - f|^2) over its atoms j != w (lj.rs:86-105; in the precision
   // variant binary32 terms accumulated in FP64), with the fast reciprocals.
@@ -780,22 +809,27 @@ struct Engine {
   // divergent branch per atom.
   SADMC_DF double lj_lane_sum(int w, double tx, double ty, double tz, double fx, double fy, double fz) {
     double acc = 0.0;
+    auto term = [&](int jr) {
+      const double xj = lx[jr], yj = ly[jr], zj = lz[jr];
+      if (PREC == 1) {
+        const float an = (float)(xj - tx), bn = (float)(yj - ty), cn = (float)(zj - tz);
+        const float ao = (float)(xj - fx), bo = (float)(yj - fy), co = (float)(zj - fz);
+        return (double)lj_pair_f32_fast(an * an + bn * bn + cn * cn) -
+               (double)lj_pair_f32_fast(ao * ao + bo * bo + co * co);
+      }
+      return lj_pair_fast(norm2(xj - tx, yj - ty, zj - tz)) - lj_pair_fast(norm2(xj - fx, yj - fy, zj - fz));
+    };
+    if constexpr (SH) {
+      const int j = lane + G * (wave_lane() / G & (KMAX - 1));
+      const bool use = (j < n) & (j != w);
+      const double t = term(use ? j : 0);
+      return shared_sum(use ? t : 0.0);
+    }
     auto slot = [&](int k) {
       const int j = lane + G * k;
       const bool use = (j < n) & (j != w);
       // slots that K may not reach read atom 0 (and are dropped)
-      const int jr = 2 * k > KMAX && j >= n ? 0 : j;
-      const double xj = lx[jr], yj = ly[jr], zj = lz[jr];
-      double t;
-      if (PREC == 1) {
-        const float an = (float)(xj - tx), bn = (float)(yj - ty), cn = (float)(zj - tz);
-        const float ao = (float)(xj - fx), bo = (float)(yj - fy), co = (float)(zj - fz);
-        t = (double)lj_pair_f32_fast(an * an + bn * bn + cn * cn) -
-            (double)lj_pair_f32_fast(ao * ao + bo * bo + co * co);
-      } else {
-        t = lj_pair_fast(norm2(xj - tx, yj - ty, zj - tz)) - lj_pair_fast(norm2(xj - fx, yj - fy, zj - fz));
-      }
-      const double na = acc + t;
+      const double na = acc + term(2 * k > KMAX && j >= n ? 0 : j);
       acc = use ? na : acc;
     };
 #pragma unroll

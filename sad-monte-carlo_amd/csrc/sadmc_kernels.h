@@ -146,7 +146,8 @@ hipError_t launch_pt(int sys, int kmax, const SetArgs &a, const PtArgs &p, int l
 // A wave takes the branches that any of its walkers takes and waits for all
 // their records, so fewer walkers per wave cost less per move as long as each
 // wave has a SIMD to itself (1024 of them): 4096 LJ13 walkers take 2.09 us a
-// move at 4 walkers a wave, 2.50 at 16 and 2.85 at 2.  The Ising walker's chain
+// move at 4 walkers a wave, 2.50 at 16 and 2.85 at 2 (1.76 at 4 with the pair
+// terms shared, lanes_to_share).  The Ising walker's chain
 // is short enough that two waves share a SIMD without loss: 4096 walkers take
 // 1.91 us a move at 2 a wave, 2.19 at 4, 2.41 at 64 and 3.4 at 1.
 static inline int walkers_per_wave(int W, int G) {
@@ -156,17 +157,27 @@ static inline int walkers_per_wave(int W, int G) {
   return per;
 }
 
+// Whether a wave of `per` walkers has the lanes to give each of a walker's G
+// one lane per atom slot (Engine's SH).  A lone wave is bound by the number of
+// instructions a move takes, and its idle lanes cost nothing: a move evaluates
+// one slot and collects the others by lane reads issued together instead of
+// evaluating KMAX slots in turn.  4096 LJ13 walkers (4 slots) 2.02 -> 1.76 us a
+// move, 64 of them 2.31 -> 1.95, 1001 WCA64 walkers (8 slots) 4.71 -> 3.60; a
+// form with the sharing chosen at run time, its lane reads in a loop, gained
+// nothing.  Where the lanes are not idle the kernel without it runs, unchanged.
+static inline bool lanes_to_share(int per, int G, int kmax) { return kmax > 1 && per * G * kmax <= 64; }
+
 // GC > 0: the set's lanes per walker as a compile-time constant.  Each of a
 // workgroup's one to four wavefronts holds `per` walkers, 64/G or fewer.
-template <int SYS, int KMAX, int PREC, int METH, int GC = 0>
+template <int SYS, int KMAX, int PREC, int METH, int GC = 0, bool SH = false>
 __global__ __launch_bounds__(256) void k_run(SetArgs a, uint64_t moves, int per) {
   extern __shared__ double lds[];
   const int G = GC ? GC : a.G;
-  const int wave = threadIdx.x / 64, group = (threadIdx.x & 63) / G;
+  const int wave = threadIdx.x / 64, group = (threadIdx.x & 63) / (SH ? G * KMAX : G);
   const int lane = threadIdx.x & (G - 1);
   const int walker = (blockIdx.x * (blockDim.x / 64) + wave) * per + group;
   double *tile = lds + (wave * per + group) * 3 * a.npad;
-  Engine<SYS, KMAX, PREC, METH, 0, GC> e;
+  Engine<SYS, KMAX, PREC, METH, 0, GC, SH> e;
   const bool held = group < per && walker < a.W;
   if (held) {
     e.load(a, walker, lane, tile);
@@ -250,6 +261,17 @@ __global__ __launch_bounds__(64) void k_energy(SetArgs a, int walker, double *ou
   if (threadIdx.x == 0) *out = e.E;
 }
 
+template <int SYS, int KMAX, int PREC, int METH, int GC>
+static void launch_run(dim3 grid, dim3 block, size_t lds, hipStream_t s, const SetArgs &a, uint64_t moves, int per) {
+  if constexpr (SYS != SYS_ISING && KMAX > 1 && GC * KMAX <= 64) {
+    if (lanes_to_share(per, a.G, KMAX)) {
+      hipLaunchKernelGGL((k_run<SYS, KMAX, PREC, METH, GC, true>), grid, block, lds, s, a, moves, per);
+      return;
+    }
+  }
+  hipLaunchKernelGGL((k_run<SYS, KMAX, PREC, METH, GC>), grid, block, lds, s, a, moves, per);
+}
+
 template <int SYS, int KMAX, int PREC, int METH>
 static hipError_t launch_t(KernelKind kk, const SetArgs &a, const LaunchArgs &la, hipStream_t s) {
   const int G = a.G;
@@ -269,22 +291,19 @@ static hipError_t launch_t(KernelKind kk, const SetArgs &a, const LaunchArgs &la
       // the lanes fixed at compile time
       if constexpr (SYS != SYS_ISING && METH == M_SAD && KMAX >= 2 && KMAX <= 8) {
         if (a.G == 4) {
-          hipLaunchKernelGGL((k_run<SYS, KMAX, PREC, METH, 4>), run_grid, run_block, run_lds, s, a, la.moves,
-                             per);
+          launch_run<SYS, KMAX, PREC, METH, 4>(run_grid, run_block, run_lds, s, a, la.moves, per);
           break;
         }
         if (a.G == 8) {
-          hipLaunchKernelGGL((k_run<SYS, KMAX, PREC, METH, 8>), run_grid, run_block, run_lds, s, a, la.moves,
-                             per);
+          launch_run<SYS, KMAX, PREC, METH, 8>(run_grid, run_block, run_lds, s, a, la.moves, per);
           break;
         }
         if (a.G == 16) {
-          hipLaunchKernelGGL((k_run<SYS, KMAX, PREC, METH, 16>), run_grid, run_block, run_lds, s, a, la.moves,
-                             per);
+          launch_run<SYS, KMAX, PREC, METH, 16>(run_grid, run_block, run_lds, s, a, la.moves, per);
           break;
         }
       }
-      hipLaunchKernelGGL((k_run<SYS, KMAX, PREC, METH>), run_grid, run_block, run_lds, s, a, la.moves, per);
+      launch_run<SYS, KMAX, PREC, METH, 0>(run_grid, run_block, run_lds, s, a, la.moves, per);
       break;
     case KK_INIT:
       hipLaunchKernelGGL((k_init<SYS, KMAX, PREC, METH>), grid, block, lds, s, a, la.e_lo);
