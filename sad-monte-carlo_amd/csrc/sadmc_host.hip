@@ -212,13 +212,18 @@ static hipError_t staging(sadmc_ctx *c) {  // under pin_mu
 // `bytes` at the device address `src` into `dst`, after everything queued on
 // the context's stream.
 static hipError_t fetch(sadmc_ctx *c, void *dst, const void *src, size_t bytes) {
-  if (bytes > kPinBytes) {
+  std::unique_lock<std::mutex> hold(c->pin_mu, std::defer_lock);
+  bool pinned = bytes <= kPinBytes;
+  if (pinned) {
+    hold.lock();
+    pinned = staging(c) == hipSuccess;
+    if (!pinned) (void)hipGetLastError();  // no pinned memory: the plain copy
+  }
+  if (!pinned) {
     const hipError_t e = hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, c->stream);
     return e != hipSuccess ? e : hipStreamSynchronize(c->stream);
   }
-  std::lock_guard<std::mutex> hold(c->pin_mu);
-  hipError_t e = staging(c);
-  if (e == hipSuccess) e = hipMemcpyAsync(c->pin, src, bytes, hipMemcpyDeviceToHost, c->stream);
+  hipError_t e = hipMemcpyAsync(c->pin, src, bytes, hipMemcpyDeviceToHost, c->stream);
   if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
   if (e == hipSuccess) std::memcpy(dst, c->pin, bytes);
   return e;
@@ -651,13 +656,10 @@ static int ensure_prop(sadmc_ctx *c) {
   return upload_weights(c, w.data());
 }
 
-int sadmc_init(sadmc_ctx *c) {
-  if (!c) return SADMC_E_ARG;
-  if (c->inited) return fail(c, SADMC_E_STATE, "already initialised");
-  if (c->sets.empty()) return fail(c, SADMC_E_STATE, "no walker sets");
-  HIPCHECK(c, hipSetDevice(c->device));
+// The device memory of every set and its walkers' from_params.
+static int init_sets(sadmc_ctx *c) {
   const size_t flag_bytes = sizeof(int32_t) * c->sets.size();
-  if (!c->d_flags) HIPCHECK(c, hipMalloc(&c->d_flags, flag_bytes));
+  HIPCHECK(c, hipMalloc(&c->d_flags, flag_bytes));
   HIPCHECK(c, hipMemsetAsync(c->d_flags, 0, flag_bytes, c->stream));
   for (auto &s : c->sets) {
     const int W = s.W, n = s.p.n;
@@ -713,6 +715,25 @@ int sadmc_init(sadmc_ctx *c) {
     HIPCHECK(c, launch(s.p.system, s.p.precision, s.p.method, s.KMAX, KK_INIT, s.args, la, c->stream));
   }
   HIPCHECK(c, hipStreamSynchronize(c->stream));
+  return SADMC_OK;
+}
+
+int sadmc_init(sadmc_ctx *c) {
+  if (!c) return SADMC_E_ARG;
+  if (c->inited) return fail(c, SADMC_E_STATE, "already initialised");
+  if (c->sets.empty()) return fail(c, SADMC_E_STATE, "no walker sets");
+  HIPCHECK(c, hipSetDevice(c->device));
+  const int rc = init_sets(c);
+  if (rc) {
+    // a start that failed leaves no memory behind: sets may be added before
+    // the next one, which allocates for as many as there are then
+    (void)hipGetLastError();  // (the next launch would report it again)
+    (void)hipStreamSynchronize(c->stream);
+    for (auto &s : c->sets) free_set(s);
+    (void)hipFree(c->d_flags);
+    c->d_flags = nullptr;
+    return rc;
+  }
   c->inited = true;
   return check_flags(c);
 }
