@@ -1270,6 +1270,8 @@ int sadmc_prop_train(sadmc_ctx *c, int32_t steps, int32_t batch, float lr, float
   }
   if (losses)
     HIPCHECK(c, fetch(c, losses, c->d_loss, sizeof(float) * steps));
+  else
+    HIPCHECK(c, hipStreamSynchronize(c->stream));
   return SADMC_OK;
 }
 

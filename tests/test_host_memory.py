@@ -69,3 +69,14 @@ def test_a_failed_start_can_be_repeated_with_more_sets(standin, kind):
     print(failed)
     """)
     assert int(out) >= 5  # every allocation of a start was the failing one once
+
+
+def test_training_has_ended_when_the_call_returns(standin):
+    """sadmc_prop_train waits for its steps whether or not the losses are asked for."""
+    _run(standin, """
+    ctx = S.Context(0)
+    ctx.prop_load_records(np.zeros((64, S.PROP_REC), np.float32))
+    for losses in (np.zeros(3, np.float32), None):
+        ctx._check(S.lib().sadmc_prop_train(ctx.h, 3, 64, 1e-3, S._p(losses)), "prop_train")
+        assert R.standin_queued() == 0, losses
+    """)
