@@ -217,7 +217,7 @@ __global__ __launch_bounds__(64) void k_plan(SetArgs a, int walker, double scale
     p.tx = e.ptx;
     p.ty = e.pty;
     p.tz = e.ptz;
-    p.e = e2;
+    p.e = some ? e2 : 0.0;  // (a move past the wall has no energy)
     p.dabse = e.pdabse;
     *out = p;
   }
