@@ -1393,8 +1393,8 @@ struct Engine {
   //
   // A move is a proposal and a visit; in between the wave recomputes the
   // energies that the proposals asked for (true) together.
-  // `step`: this move's lane in rs_wave (the same in the whole wave).
-  SADMC_DF bool propose(int step) {
+  // `rs`: sqrt(1 / moves), this move counted.
+  SADMC_DF bool propose(double rs) {
     bool regrow = false;
     tm += 1.0;
     if (METH == M_SAD) tl_now = false;
@@ -1427,15 +1427,6 @@ struct Engine {
       }
       g_next += 1;
       gpre = gamma_now();
-    }
-    double rs;
-    if (__builtin_expect(rs_same, 1)) {
-      const uint64_t b = __builtin_bit_cast(uint64_t, rs_wave);
-      const uint32_t lo = __builtin_amdgcn_readlane((int)(uint32_t)b, step);
-      const uint32_t hi = __builtin_amdgcn_readlane((int)(uint32_t)(b >> 32), step);
-      rs = __builtin_bit_cast(double, ((uint64_t)hi << 32) | lo);
-    } else {
-      rs = sqrt(1.0 / tm);
     }
     double e2 = e1;
     bool go = plan_move(tscale, usc, e2);
@@ -1561,6 +1552,17 @@ struct Engine {
     rs_same = __ballot(1) == ~0ULL && !__any((status == 0) & (tm != t));
     rs_wave = sqrt(1.0 / (t + (double)((threadIdx.x & 63) + 1)));
   }
+  // The one of this move, `step` moves on (the same in the whole wave).  Only
+  // where the wave's lanes all run: the lane read may belong to a walker that
+  // has stopped or to no walker, and what such a lane holds of rs_wave is
+  // certain only outside the branches it sits out.
+  SADMC_DF double root(int step) const {
+    if (__builtin_expect(!rs_same, 0)) return sqrt(1.0 / (tm + 1.0));
+    const uint64_t b = __builtin_bit_cast(uint64_t, rs_wave);
+    const uint32_t lo = __builtin_amdgcn_readlane((int)(uint32_t)b, step);
+    const uint32_t hi = __builtin_amdgcn_readlane((int)(uint32_t)(b >> 32), step);
+    return __builtin_bit_cast(double, ((uint64_t)hi << 32) | lo);
+  }
 
   SADMC_DF void run(uint64_t nmoves) {
     // (the loop's exit is the wave's, not a walker's: a divergent exit makes
@@ -1569,8 +1571,9 @@ struct Engine {
     for (uint64_t k = 0; k < nmoves && __any(status == 0); k++) {
       const int step = (int)(k & 63);
       if (step == 0) next_roots();
+      const double rs = root(step);
       bool trip = false;
-      if (__builtin_expect(status == 0, 1)) trip = propose(step);
+      if (__builtin_expect(status == 0, 1)) trip = propose(rs);
       if (__builtin_expect(__any(trip), 0)) {
         full_energies(trip);
         if (trip) {
