@@ -1393,7 +1393,7 @@ struct Engine {
   //
   // A move is a proposal and a visit; in between the wave recomputes the
   // energies that the proposals asked for (true) together.
-  // `rs`: sqrt(1 / moves), this move counted.
+  // `rs`: sqrt(1 / moves), this move counted, where rs_same.
   SADMC_DF bool propose(double rs) {
     bool regrow = false;
     tm += 1.0;
@@ -1428,6 +1428,7 @@ struct Engine {
       g_next += 1;
       gpre = gamma_now();
     }
+    if (__builtin_expect(!rs_same, 0)) rs = sqrt(1.0 / tm);
     double e2 = e1;
     bool go = plan_move(tscale, usc, e2);
     acc_rate *= 1.0 - rs;
@@ -1557,7 +1558,6 @@ struct Engine {
   // has stopped or to no walker, and what such a lane holds of rs_wave is
   // certain only outside the branches it sits out.
   SADMC_DF double root(int step) const {
-    if (__builtin_expect(!rs_same, 0)) return sqrt(1.0 / (tm + 1.0));
     const uint64_t b = __builtin_bit_cast(uint64_t, rs_wave);
     const uint32_t lo = __builtin_amdgcn_readlane((int)(uint32_t)b, step);
     const uint32_t hi = __builtin_amdgcn_readlane((int)(uint32_t)(b >> 32), step);
