@@ -1440,7 +1440,11 @@ struct Engine {
         lo = E < lo ? E : lo;
         hi = E > hi ? E : hi;
       }
+      // (also for a walker that the energy check above has stopped)
+      const int32_t stopped = status;
+      status = 0;
       prepare_for_range(lo, hi);
+      status = status ? status : stopped;
     }
     i1 = go ? cur_i : i1;
     const int32_t i2 = e_index(go ? e2 : e1);
