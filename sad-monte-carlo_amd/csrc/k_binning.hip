@@ -80,7 +80,7 @@ struct BinWalker {
   sadmc_bbin *B;  // this walker's window of bins
   BC<CT> *bc;     // [kBinStats] in LDS
   int lane, G;
-  double tm;  // the move count, whole and exact
+  double tm;  // the move count, whole and exact (these walkers start at 0: no state is uploaded)
   SADMC_DF uint64_t moves() const { return (uint64_t)tm; }
   uint64_t accepted;
   double acc_rate, tscale, usc;

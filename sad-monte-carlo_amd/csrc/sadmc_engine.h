@@ -157,9 +157,8 @@ struct Engine {
   // EnergyMC scalars
   uint64_t s0, s1;
   double E, err;
-  uint64_t accepted;
-  double tm;  // the move count, whole and exact (below 2^53)
-  SADMC_DF uint64_t moves() const { return (uint64_t)tm; }
+  uint64_t moves, accepted;
+  double tm;  // (double)moves, kept exact by +1.0 steps
   double acc_rate, tscale, usc;
   double bmin;
   int32_t base, len;
@@ -168,13 +167,14 @@ struct Engine {
   uint64_t epoch;
   int32_t bulk, status, method;
   double btop;  // bmin + width * len, the upper edge of the bins
-  // SAD (tF and N_s are whole and exact); rtF, rNs = 1 / tF, 1 / N_s and
+  // SAD; rtF, rNs = 1 / tF, 1 / N_s and
   // gzero (gamma is 0) follow lam, tF and N_s, which change rarely; tl_now:
   // tL was set in this move; tmax: the largest t_found in the range.  What a
   // walker below too_lo needs each move is here too: one such walker, which
   // can stay there for a whole launch, holds up its wave and so the launch.
   // tL and WCA's has_pressure, only ever written, stay in the walker's record.
-  double too_lo, too_hi, lam, min_T, tF, Ns, rtF, rNs, lnw_lo, lnw_hi, tmax;
+  double too_lo, too_hi, lam, min_T, rtF, rNs, lnw_lo, lnw_hi;
+  uint64_t tF, Ns, tmax;
   bool gzero, tl_now;
   uint64_t highest;
   int32_t ilo, ihi;
@@ -193,7 +193,7 @@ struct Engine {
   uint64_t c_rt, c_vep;
   int32_t from_i;  // the bin this move started in
   // periodic triggers
-  double next_check, next_press;  // in moves
+  uint64_t next_check, next_press;
   // pending move
   int32_t pw;
   double ptx, pty, ptz, pe, pdabse;
@@ -255,7 +255,8 @@ struct Engine {
     s1 = w.rng[1];
     E = w.E;
     err = w.error;
-    tm = (double)w.moves;
+    moves = w.moves;
+    tm = (double)moves;
     accepted = w.accepted_moves;
     acc_rate = w.acceptance_rate;
     tscale = w.translation_scale;
@@ -273,9 +274,9 @@ struct Engine {
       too_hi = w.too_hi;
       lam = w.latest_parameter;
       min_T = w.min_T;
-      tmax = (double)w.tmax;
-      tF = (double)w.tF;
-      Ns = (double)w.num_states;
+      tmax = w.tmax;
+      tF = w.tF;
+      Ns = w.num_states;
       highest = w.highest_hist;
     }
     if (METH == M_SAMC || METH == M_WL) t0 = w.t0;
@@ -314,10 +315,10 @@ struct Engine {
         w.too_lo = too_lo;
         w.too_hi = too_hi;
         w.latest_parameter = lam;
-        w.tF = (uint64_t)tF;
-        w.num_states = (uint64_t)Ns;
+        w.tF = tF;
+        w.num_states = Ns;
         w.highest_hist = highest;
-        w.tmax = (uint64_t)tmax;
+        w.tmax = tmax;
       }
       if (METH == M_SAMC || METH == M_WL) w.t0 = t0;
       if (METH == M_WL) {
@@ -339,7 +340,7 @@ struct Engine {
       w.rng[1] = s1;
       w.E = E;
       w.error = err;
-      w.moves = moves();
+      w.moves = moves;
       w.accepted_moves = accepted;
       w.acceptance_rate = acc_rate;
       w.translation_scale = tscale;
@@ -466,10 +467,10 @@ struct Engine {
   SADMC_DF void reset_checks() {
     if (SYS != SYS_ISING) {
       uint64_t P = args().refresh > 0 ? (uint64_t)args().refresh : (uint64_t)len * (uint64_t)len * 1000ULL;
-      next_check = (double)((moves() / P + 1) * P);
+      next_check = (moves / P + 1) * P;
       if (SYS == SYS_WCA) {
         uint64_t Q = (uint64_t)n * (uint64_t)n;
-        next_press = (double)((moves() / Q + 1) * Q);
+        next_press = (moves / Q + 1) * Q;
       }
     }
   }
@@ -509,7 +510,7 @@ struct Engine {
     if (status == 0 && (front || (grew && !indices_valid()))) refresh_indices(plo, phi);
     if (status == 0 && (front || grew) && SYS != SYS_ISING && args().refresh <= 0) {
       uint64_t P = (uint64_t)len * (uint64_t)len * 1000ULL;
-      next_check = (double)((moves() / P + 1) * P);
+      next_check = (moves / P + 1) * P;
     }
   }
 
@@ -1052,24 +1053,24 @@ struct Engine {
   // RN(t y) is within two units of the quotient, the first residual step
   // brings it to a faithful one, and with a faithful quotient the second
   // gives the correctly rounded one (Markstein 1990), which is the division's.
-  // The operands are whole numbers below 2^53 (b >= 1; otherwise gamma is 0),
-  // so nothing over- or underflows.
+  // The operands lie between 1/2 and 2^64 (b; otherwise gamma is 0), so nothing
+  // over- or underflows.
   SADMC_DF static double quot(double a, double b, double y) {
     double q = a * y;
     q = __builtin_fma(__builtin_fma(-b, q, a), y, q);
     return __builtin_fma(__builtin_fma(-b, q, a), y, q);
   }
   SADMC_DF double sad_gamma(double t) const {
-    const double q = quot(t, tF, rtF);
-    const double g = (lam + q) / (lam + quot(t, Ns, rNs) * q);
+    const double q = quot(t, (double)tF, rtF);
+    const double g = (lam + q) / (lam + quot(t, (double)Ns, rNs) * q);
     return gzero ? 0.0 : g;
   }
   // After a change of lam, tF or Ns (during move tm): the reciprocals, and
   // the gammas of the moves from tm on that the lanes hold.
   SADMC_DF void gamma_changed() {
-    rtF = 1.0 / tF;
-    rNs = 1.0 / Ns;
-    gzero = lam * tF * Ns == 0.0;
+    rtF = 1.0 / (double)tF;
+    rNs = 1.0 / (double)Ns;
+    gzero = lam * (double)tF * (double)Ns == 0.0;
     g_lane = sad_gamma(tm + (double)(lane - (g_next - 1)));
   }
   SADMC_DF double gamma_now() const { return G == 1 ? g_lane : __shfl(g_lane, g_next - 1, G); }
@@ -1146,7 +1147,7 @@ struct Engine {
     if (METH == M_SAD) {
       if (__builtin_expect(found, 0) && e2 < too_hi && e2 > too_lo) {
         lam = (too_hi - too_lo) / min_T;
-        Ns += 1.0;
+        Ns += 1;
         set_tL();
         gamma_changed();
         gpre = gamma_now();
@@ -1175,7 +1176,7 @@ struct Engine {
   }
   SADMC_DF void set_tL() {
     tl_now = true;
-    rec().tL = moves();
+    rec().tL = moves;
   }
   SADMC_DF void tmax_scan(int32_t a, int32_t b) {
     const uint64_t *TF = tfound();
@@ -1185,7 +1186,7 @@ struct Engine {
       m = t > m ? t : m;
     }
     m = group_max_u64(m);
-    tmax = (double)m > tmax ? (double)m : tmax;
+    tmax = m > tmax ? m : tmax;
   }
 
   // energy.rs:514-636 for the current bin (logical i = cur_i).
@@ -1229,7 +1230,7 @@ struct Engine {
             cnt += c_hist != 0 ? 1u : 0u;
           }
         }
-        Ns += (double)cnt;
+        Ns += cnt;
         __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
         lam = (E - too_lo) / min_T;
         set_tL();
@@ -1273,7 +1274,7 @@ struct Engine {
             cnt += c_hist != 0 ? 1u : 0u;
           }
         }
-        Ns += (double)cnt;
+        Ns += cnt;
         __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
         lam = (too_hi - E) / min_T;
         set_tL();
@@ -1290,7 +1291,7 @@ struct Engine {
     }
     if (tl_now && status == 0 && (ilo >= len || ihi >= len)) status = SADMC_WS_INDEX;
     if (tl_now && status == 0) {
-      const double old_tF = tF;
+      const uint64_t old_tF = tF;
       tF = tmax;
       if (old_tF != tF && args().move_plan == SADMC_ACCEPTANCE_RATE) {
         double s = acc_rate / args().move_param;
@@ -1396,13 +1397,14 @@ struct Engine {
   // `rs`: sqrt(1 / moves), this move counted, where rs_same.
   SADMC_DF bool propose(double rs) {
     bool regrow = false;
+    moves += 1;
     tm += 1.0;
     if (METH == M_SAD) tl_now = false;
-    if (SYS != SYS_ISING && __builtin_expect(tm == next_check, 0)) {
+    if (SYS != SYS_ISING && __builtin_expect(moves == next_check, 0)) {
       const double egood = full_energy();
       if (args().refresh > 0) {
         E = egood;
-        next_check += (double)args().refresh;
+        next_check += (uint64_t)args().refresh;
         // the refreshed energy may lie in another bin than the tracked one
         // (move_once indexes the bins by the energy itself, energy.rs:904-974),
         // or past the window's edge by the FP32 drift: the window then grows
@@ -1415,7 +1417,7 @@ struct Engine {
         }
       } else {
         verify_energy(egood);
-        next_check += (double)((uint64_t)len * (uint64_t)len * 1000ULL);
+        next_check += (uint64_t)len * (uint64_t)len * 1000ULL;
       }
     }
     const double e1 = E;
@@ -1503,11 +1505,11 @@ struct Engine {
     const int32_t i = cur_i;
     const int32_t p = cur_p;
     if (__builtin_expect(c_hist == 0, 0)) {
-      tfound()[p] = moves();
-      if (METH == M_SAD && i >= ilo && i <= ihi) tmax = tm;
+      tfound()[p] = moves;
+      if (METH == M_SAD && i >= ilo && i <= ihi) tmax = moves;
     }
     c_hist += 1;
-    if (SYS == SYS_WCA && args().collect_pressure && __builtin_expect(tm == next_press, 0)) {
+    if (SYS == SYS_WCA && args().collect_pressure && __builtin_expect(moves == next_press, 0)) {
       const double pv = pressure();
       PExtra &x = args().extra[(int64_t)wk * args().cap + p];
       rec().has_pressure = 1;
@@ -1515,7 +1517,7 @@ struct Engine {
         x.count += 1;
         x.total += pv;
       }
-      next_press += (double)n * (double)n;
+      next_press += (uint64_t)n * (uint64_t)n;
     }
     if (METH == M_SAD) {
       update_sad(En, i);
@@ -1638,7 +1640,7 @@ struct Engine {
     max_S_index = 0;
     epoch = 1;
     bulk = 0;
-    tm = 0.0;
+    moves = 0;
     accepted = 0;
     acc_rate = 0.5;
     tscale = args().move_plan == SADMC_TRANSLATION_SCALE ? args().move_param : 0.05;
