@@ -91,3 +91,41 @@ def test_neighbours_at_different_move_numbers(gpu_ctx_factory, kw, geom, walkers
         c.close()
     assert sm.tobytes() == np.where(odd, sb, sa).tobytes()
     assert bm.tobytes() == np.where(odd[:, None], bb, ba).tobytes()
+
+
+@pytest.mark.parametrize("kw,geom,sizes", [
+    pytest.param(dict(LJ13, method=S.WL, method_param=0.0, has_min_e=1, min_e=-44.0), 2.5, (3, 2100, LJ13_FULL),
+                 id="lj13-wl"),
+    pytest.param(dict(LJ13, method=S.INV_T_WL, method_param=0.0, has_min_e=1, min_e=-44.0), 2.5, (3, 2100, LJ13_FULL),
+                 id="lj13-inv-t-wl"),
+    pytest.param(dict(LJ13, method=S.CANONICAL, method_param=0.3), 2.5, (3, 2100, LJ13_FULL), id="lj13-canonical"),
+    pytest.param(dict(LJ13, method=S.CANONICAL, method_param=0.2, precision=S.FP32_PAIRS, refresh=256), 2.5,
+                 (3, 2100, LJ13_FULL), id="lj13-fp32-canonical"),
+    pytest.param(dict(LJ13, precision=S.FP32_PAIRS, refresh=256), 2.5, (3, 2100, LJ13_FULL), id="lj13-fp32-sad"),
+    pytest.param(dict(system=S.WCA, n=32, lanes=8, method=S.CANONICAL, method_param=1.0, move_param=0.05,
+                      energy_bin=0.2, has_max_e=1, max_e=80.0, collect_pressure=1), 3.6, (3, 1100, 8 * 1024 + 10),
+                 id="wca32-canonical"),
+    pytest.param(dict(system=S.ISING, n=8, ising_init=1, method=S.INV_T_WL, has_min_e=1, min_e=-116.0, has_max_e=1,
+                      max_e=116.0), None, (3, 4200, ISING_FULL), id="ising-inv-t-wl"),
+])
+def test_methods_do_not_depend_on_the_wave(gpu_ctx_factory, kw, geom, sizes):
+    """The first walkers of small and full sets, and the small set's against the oracle."""
+    print("case", kw["system"], kw["method"], flush=True)
+    sp = S.make_params(**kw)
+    moves, ref = (700, 600), None
+    for walkers in sizes:
+        ctx = gpu_ctx_factory()
+        s = ctx.add_set(sp, np.arange(walkers, dtype=np.uint64) + 300, geom=geom)
+        ctx.init()
+        for m in moves:
+            ctx.run(m)
+        st, _ = ctx.download_raw(s, with_bins=False)
+        bins = [ctx.bins(s, w) for w in range(3)]
+        got = (st[:3].tobytes(), [{k: v.tobytes() for k, v in b.items()} for b in bins])
+        if ref is None:
+            ref = got
+            orcs = run_oracles([oracle_params(sp, w + 300, geom or 0.0) for w in range(3)], sum(moves))
+            for w in range(3):
+                compare_walker(ctx.state(s, w), bins[w], orcs[w], sp.method, label=f"walker {w}")
+        ctx.close()
+        assert got == ref, f"{walkers} walkers"
