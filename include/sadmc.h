@@ -162,7 +162,10 @@ const char *sadmc_last_error(const sadmc_ctx *ctx);
 int sadmc_add_set(sadmc_ctx *ctx, const sadmc_set_params *p, int32_t n_walkers, const uint64_t *seeds,
                   const double *geom, const double *coords, const int8_t *spins, int32_t *set_id);
 /* Allocate device state, upload, and run from_params on the device (initial
- * energy, optional greedy descent below max_e, one-bin histogram). */
+ * energy, optional greedy descent below max_e, one-bin histogram).  A start
+ * that fails for want of memory (SADMC_E_HIP) leaves none behind: sets may
+ * still be added, and the call repeated.  Its check of the walkers also makes
+ * the context's pinned staging for small reads (64 KiB, about 0.1 ms, once). */
 int sadmc_init(sadmc_ctx *ctx);
 
 /* ---- the hot path: K x move_once for every walker (energy.rs:904-974) - */
@@ -229,7 +232,7 @@ int sadmc_check_recip_f32(int device, int32_t what, uint64_t lo, uint64_t hi, ui
 
 /* ---- single-walker pair for parity tests: MovableSystem::plan_move and
  * ConfirmSystem::confirm (system/mod.rs:101-120).  plan_move consumes the
- * walker's RNG exactly as inside move_once; *some = 0 means None. */
+ * walker's RNG exactly as inside move_once; *some = 0 means None (*e_new is then 0). */
 int sadmc_plan_move(sadmc_ctx *ctx, int32_t set, int32_t walker, double scale, double *e_new, int32_t *some);
 int sadmc_confirm(sadmc_ctx *ctx, int32_t set, int32_t walker);
 
@@ -255,7 +258,8 @@ int sadmc_prop_records(sadmc_ctx *ctx, float *out, int64_t max_records, int64_t 
 int sadmc_prop_load_records(sadmc_ctx *ctx, const float *records, int64_t count);
 /* Mean loss and gradient over records [first, first+count) (cyclic). */
 int sadmc_prop_gradient(sadmc_ctx *ctx, int64_t first, int32_t count, float *grad, float *loss);
-/* `steps` Adam steps on consecutive minibatches; losses[k] = step k's loss. */
+/* `steps` Adam steps on consecutive minibatches; losses[k] = step k's loss
+ * (losses may be NULL).  Returns when the steps have ended. */
 int sadmc_prop_train(sadmc_ctx *ctx, int32_t steps, int32_t batch, float lr, float *losses);
 
 /* ---- mean entropy on the device (plotting/parse-binning.py:150-171) ---

@@ -331,9 +331,12 @@ hipError_t launch_entropy_range(const sadmc_walker_state *ws, int W, double widt
   return hipGetLastError();
 }
 
+// Chunks of walkers: 2048 pieces of 256 bins of a chunk, which k_entropy_bins
+// takes 256 * kBinsPerLane at a time (two: 1024 blocks, 4 per CU).  The count
+// is part of the result: the sums are added chunk by chunk.
 int entropy_chunks(int W, int64_t ng) {
   const int64_t blocks = (ng + 255) / 256;
-  int64_t c = (2048 + blocks - 1) / blocks;  // about 8 blocks per CU
+  int64_t c = (2048 + blocks - 1) / blocks;
   if (c > 64) c = 64;
   if (c > W) c = W;
   return c < 1 ? 1 : (int)c;

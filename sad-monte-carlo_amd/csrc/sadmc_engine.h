@@ -1,6 +1,6 @@
-// Device walker engine: one reference `EnergyMC::move_once`
-// (src/mc/energy.rs:904-974) per call, for a group of G lanes that share one
-// walker.
+// Device walker engine: the reference's `EnergyMC::move_once`
+// (src/mc/energy.rs:904-974), as a proposal and a visit, for a group of G lanes
+// that share one walker.
 //
 // Layout.  Every lane of a group holds the walker's hot scalar state in
 // registers (identical values: all lanes execute the same bookkeeping, so no

@@ -160,8 +160,8 @@ struct sadmc_ctx {
   size_t ent_bytes = 0;
   // the walker sets' stop flags, one each, so that a sync reads them at once
   int32_t *d_flags = nullptr;
-  // pinned staging for small reads (kPinBytes, made on first use); one reader
-  // at a time
+  // pinned staging for small reads (kPinBytes), made once, by the first read
+  // (the stop flags' in sadmc_init); one reader at a time
   char *pin = nullptr;
   std::mutex pin_mu;
 };

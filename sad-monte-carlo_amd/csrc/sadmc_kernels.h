@@ -145,11 +145,13 @@ hipError_t launch_pt(int sys, int kmax, const SetArgs &a, const PtArgs &p, int l
 // that leaves SIMDs without a wave; then half as many, and so on down to one.
 // A wave takes the branches that any of its walkers takes and waits for all
 // their records, so fewer walkers per wave cost less per move as long as each
-// wave has a SIMD to itself (1024 of them): 4096 LJ13 walkers take 2.09 us a
-// move at 4 walkers a wave, 2.50 at 16 and 2.85 at 2 (1.76 at 4 with the pair
-// terms shared, lanes_to_share).  The Ising walker's chain
-// is short enough that two waves share a SIMD without loss: 4096 walkers take
-// 1.91 us a move at 2 a wave, 2.19 at 4, 2.41 at 64 and 3.4 at 1.
+// wave has a SIMD to itself (1024 of them): 4096 LJ13 walkers take 2.13 us a
+// move at 4 walkers a wave, 2.28 at 8, 2.41 at 16 and 2.61 at 2 (1.89 at 4
+// with the pair terms shared, lanes_to_share); 2048 of them 1.75 at 2 a wave,
+// shared, 1.83 at 4 and 1.99 at 1.  Two waves of Ising walkers share a SIMD
+// with little loss: 4096 walkers take 1.79 us a move at 2 a wave, 1.69 at 4,
+// 2.10 at 64 and 3.16 at 1; 8192 of them 1.97 at 4, 1.91 at 8, 2.06 at 64.
+// (Moves 60000 on, the whole set's time.)
 static inline int walkers_per_wave(int W, int G) {
   const int target = G == 1 ? 2048 : 1024;
   int per = 64 / G;
@@ -161,8 +163,8 @@ static inline int walkers_per_wave(int W, int G) {
 // one lane per atom slot (Engine's SH).  A lone wave is bound by the number of
 // instructions a move takes, and its idle lanes cost nothing: a move evaluates
 // one slot and collects the others by lane reads issued together instead of
-// evaluating KMAX slots in turn.  4096 LJ13 walkers (4 slots) 2.02 -> 1.76 us a
-// move, 64 of them 2.31 -> 1.95, 1001 WCA64 walkers (8 slots) 4.71 -> 3.60; a
+// evaluating KMAX slots in turn.  4096 LJ13 walkers (4 slots) 2.13 -> 1.89 us a
+// move, 64 of them 1.88 -> 1.56, 1001 WCA64 walkers (8 slots) 4.56 -> 3.41; a
 // form with the sharing chosen at run time, its lane reads in a loop, gained
 // nothing.  Where the lanes are not idle the kernel without it runs, unchanged.
 static inline bool lanes_to_share(int per, int G, int kmax) { return kmax > 1 && per * G * kmax <= 64; }
